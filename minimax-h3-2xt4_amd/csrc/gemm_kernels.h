@@ -142,36 +142,6 @@ __device__ __forceinline__ void store_quadrant(const GemmParams& p, v4i (&acc)[8
   store_tiles<EPI, OUT, 0>(p, acc, as, mw, nw, fr, fc);
 }
 
-// The same for a 4x4 grid of 32x32 tiles (v_mfma_i32_32x32x32_i8 layout):
-// lane (fr = lane % 32, fh = lane / 32) holds, for register group g = 0..3,
-// C[m][n..n+3] with m = mw + 32 mb + fr and n = nw + 32 nb + 8 g + 4 fh.
-// Used for partial tiles at the matrix edge.
-template <int EPI, int OUT, int T>
-__device__ __forceinline__ void store_tiles32(const GemmParams& p, v16i (&acc)[4][4], const float (&as)[4], int mw,
-                                              int nw, int fr, int fh) {
-  constexpr int NB = T / 16, MB = (T / 4) % 4, G = T % 4;
-  const int n = nw + NB * 32 + 8 * G + 4 * fh;
-  const int m = mw + MB * 32 + fr;
-  const int valid = min(4, p.n - n);
-  if (valid > 0 && m < p.m) {
-    const int c[4] = {acc[NB][MB][4 * G], acc[NB][MB][4 * G + 1], acc[NB][MB][4 * G + 2], acc[NB][MB][4 * G + 3]};
-    epilogue4<EPI, OUT>(p, m, n, valid, c, as[MB]);
-  }
-  if constexpr (T + 1 < 64) store_tiles32<EPI, OUT, T + 1>(p, acc, as, mw, nw, fr, fh);
-}
-
-template <int EPI, int OUT>
-__device__ __forceinline__ void store_quadrant32(const GemmParams& p, v16i (&acc)[4][4], int mw, int nw, int fr,
-                                                 int fh) {
-  float as[4];
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
-    const int m = mw + mb * 32 + fr;
-    as[mb] = (EPI != kEpiInt32 && m < p.m) ? p.row_scale[m] : 0.0f;
-  }
-  store_tiles32<EPI, OUT, 0>(p, acc, as, mw, nw, fr, fh);
-}
-
 // Output element bits of one accumulator (storage dtype OUT; with a residual
 // the FP16 branch is stored and the residual is added on write-out).
 template <int EPI, int OUT>
@@ -249,7 +219,7 @@ __device__ __forceinline__ int readout_col(int nw, int h, int lane) {
 // reads, and the next pass's writes may issue before this pass's reads
 // return.
 template <int EPI, int OUT, int FLAGS, bool INTERIOR, int NB = 4>
-__device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v16i (&acc)[NB][4],
+__device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i (&acc)[2 * NB][8],
                                                         const float (&wsc)[2][8], const float (&bsc)[2][8],
                                                         const float (&as)[4], const int (&lbl)[4], int mw, int nw,
                                                         int lane, int8_t* stage, int64_t out_off) {
@@ -258,7 +228,7 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v16
   constexpr bool has_bias = (FLAGS & kWithBias) != 0;
   constexpr bool has_res = (FLAGS & kWithResidual) != 0;
   constexpr bool has_gate = (FLAGS & kWithGate) != 0;
-  const int fr = lane & 31, fh = lane >> 5;
+  const int fr = lane & 15, fh = lane >> 4;
   const int orow = lane / R::LPR, ocol = (lane % R::LPR) * R::CPL;
   // The FP16 residual rows of pass `pass` (this lane's read-out columns).
   // Without the gate, pass + 1's rows are loaded while pass is dequantized,
@@ -346,18 +316,14 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v16
       gate_one = __builtin_amdgcn_ballot_w64(lbl[mb] != lab0) == 0;
       if (gate_one) load_gate(lab0, gv);
     }
-    // acc[nb][mb] group g holds columns 32 nb + 8 g + 4 fh + [0, 4) of row fr.
+    // acc[nb][mb] holds columns 16 nb + 4 fh + [0, 4) of row 16 mb + fr.
 #pragma unroll
-    for (int nbl = 0; nbl < 2; ++nbl)
+    for (int ml = 0; ml < 2; ++ml)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int nb = min(2 * h + nbl, NB - 1);
-        if (NB == 4 || 2 * h + nbl < NB) {
-          const int chunk = nbl * 8 + 2 * g + fh;
-          *reinterpret_cast<v4i*>(stage + fr * RB + ((chunk ^ (fr & 15)) << 4)) =
-              v4i{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
-        }
-      }
+      for (int nl = 0; nl < 4; ++nl)
+        if (4 * h + nl < 2 * NB)
+          *reinterpret_cast<v4i*>(stage + (16 * ml + fr) * RB + (((4 * nl + fh) ^ fr) << 4)) =
+              acc[min(4 * h + nl, 2 * NB - 1)][2 * mb + ml];
     asm volatile("" ::: "memory");
     // Row scales of the lane's read-out rows (from the lanes holding them in
     // the MFMA layout), issued with the slice reads so one wait covers both.
@@ -538,11 +504,10 @@ __device__ __forceinline__ void load_rope_freqs(const void* frow, int p0, int si
 // slice after the normalized values replace the accumulators there. Rows
 // past m are not stored (their rotation matrices are those of row m - 1).
 template <int EPI, int FQ, bool PAIRS>
-__device__ __forceinline__ void store_quadrant_rope(const GemmParams& p, v16i (&acc)[4][4], const float (&wsc)[2][8],
+__device__ __forceinline__ void store_quadrant_rope(const GemmParams& p, v4i (&acc)[8][8], const float (&wsc)[2][8],
                                                     const float (&as)[4], int mw, int nw, int lane, int8_t* stage) {
   constexpr int RB = 512;   // 128 four-byte values per staged row
   constexpr int FES = FQ == kF32 ? 4 : 2;
-  const int fr = lane & 31, fh = lane >> 5;
   const int rq = lane >> 4, t = lane & 15;
   const int d0 = 8 * t, half = p.rope_half;
   const bool rotated = d0 < p.rope_rot;
@@ -555,18 +520,10 @@ __device__ __forceinline__ void store_quadrant_rope(const GemmParams& p, v16i (&
   for (int pass = 0; pass < 8; ++pass) {   // unrolled: acc is indexed by pass
     const int mb = pass >> 1, hh = pass & 1;
     const int mrow = mw + mb * 32 + 16 * hh;
-    // acc[nb][mb] group g holds columns 32 nb + 8 g + 4 fh + [0, 4) of row fr.
-    if ((fr >> 4) == hh) {
-      const int r = fr & 15;
+    // acc[nb][pass] holds columns 16 nb + 4 rq + [0, 4) of the pass's row t.
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int chunk = 8 * nb + 2 * g + fh;
-          *reinterpret_cast<v4i*>(stage + r * RB + ((chunk ^ r) << 4)) =
-              v4i{acc[nb][mb][4 * g], acc[nb][mb][4 * g + 1], acc[nb][mb][4 * g + 2], acc[nb][mb][4 * g + 3]};
-        }
-    }
+    for (int nb = 0; nb < 8; ++nb)
+      *reinterpret_cast<v4i*>(stage + t * RB + (((4 * nb + rq) ^ t) << 4)) = acc[nb][pass];
     asm volatile("" ::: "memory");
     float arow[4];
     int c[4][8];
@@ -790,34 +747,45 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
 // 32 KB slots, one operand tile of one stage each: unit h (the A tile of
 // stage h / 2 for even h, its B tile for odd h) lives in slot h % 5. While
 // stage g computes from units 2g and 2g + 1, units 2g + 2 .. 2g + 4 stream
-// in; the barrier at the end of stage g releases two slots for units 2g + 5
-// and 2g + 6. An A unit is NA = BM / 32 DMA instructions per wave and a B
-// unit JB = BN / 32 (8 rows each): 8 and 8 for 256 x 256 tiles, 8 and 6 for
-// 256 x 192, 4 and 8 for 128 x 256. The K = 32 sub-steps spread a stage's
-// NA + JB instructions one after each MFMA row, so the address unit never
-// queues a burst in front of the MFMAs. A tile's epilogue stages its
-// accumulators through the B slot of its last stage, whose next unit is
-// issued only during the next stage.
+// in; the barrier in the middle of stage g (once its last fragments are in
+// registers) releases two slots for units 2g + 5 and 2g + 6. An A unit is
+// NA = BM / 32 DMA instructions per wave and a B unit JB = BN / 32 (8 rows
+// each): 8 and 8 for 256 x 256 tiles, 8 and 6 for 256 x 192, 4 and 8 for
+// 128 x 256. A tile's epilogue stages its accumulators through the B slot of
+// its last stage, whose next unit is issued only during the next stage.
 //
 // 128 x 256 tiles (a 48 KB stage, whose A tile would fill half a slot) take
 // a ring of three whole stages instead: stage g computes from slot g mod 3
 // while stage g + 1 lands and stage g + 2 streams into the slot stage g - 1
 // released, so two stages are in flight.
 //
+// What bounds it: at the large shapes the board's power. The products run on
+// 16x16x64 MFMAs, which sustain 4260 TOPS (2.08 GHz) from one wave per SIMD
+// on Gaussian int8 data where 32x32x32 sustains 3590 (1.73 GHz; MFMAs
+// alone), having half the accumulator traffic per product. The rest of the
+// energy feeds the operands. Against 32x32x32 with four-MFMA rows and the
+// reads and DMA bunched between them, timed in turn on one box: FC1
+// 16384x16384x3072 703 -> 644 us, FC2 16384x3072x8192 323 -> 295, QKV
+// 53504x9216x3072 1287 -> 1181, 4096x3072x3072 38.2 -> 34.1, 512x14336x4096
+// 31.8 -> 27.9 (of which the spreading of reads and DMA one to an MFMA is
+// 1..4%). MFMA pipes busy 0.65 at 1.84 GHz (0.64 at 1.74 before). Raster
+// groups of 4 row tiles instead of 8 (A rows that stay in an XCD's L2) were
+// within 1% either way, and non-temporal loads of either operand 5..50%
+// slower.
+//
 // The waits count outstanding loads instead of draining them: before each
 // stage barrier vmcnt(NA) lgkmcnt(0) (the next stage landed; only the A unit
 // issued after it may still be in flight; this wave's fragment reads of the
-// stage returned), and before the epilogue vmcnt(NA + JB / 2) (the tile's
-// scale and bias loads, issued before its K loop, have landed; only the
-// next stage's A unit and half its B unit are younger): 8 / 12 for 256 x 256
-// and 8 / 11 for 256 x 192 tiles. The three-stage ring waits vmcnt(NA +
-// 3 JB / 4) = 10 at the barrier (stage g + 2's instructions issued so far
-// are younger) and vmcnt(NA + JB) = 12 before the epilogue. Loads return in
-// order, so a count is exact whenever at least that many younger loads exist.
+// stage returned), and before the epilogue vmcnt(NA + JB) (the tile's scale
+// and bias loads, issued before its K loop, have landed; only the two units
+// its last stage issued are younger): 8 / 16 for 256 x 256 and 8 / 14 for
+// 256 x 192 tiles. The three-stage ring waits vmcnt(NA + JB) = 12 at both.
+// Loads return in order, so a count is exact whenever at least that many
+// younger loads exist.
 //
 // LDS rows are 128 bytes: 16-byte chunk c of row r sits at physical chunk
 // c ^ ((r >> 1) & 7), which keeps both the DMA writes (lane i writes bytes
-// [16 i, 16 i + 16) of its instruction's 1 KB) and the fragment reads (32
+// [16 i, 16 i + 16) of its instruction's 1 KB) and the fragment reads (16
 // rows x one chunk per 16-lane group) free of bank conflicts. A DMA lane
 // therefore loads the logical chunk that lands on its physical slot.
 constexpr int kSK = 128;                    // K bytes per stage
@@ -841,6 +809,44 @@ __device__ __forceinline__ void block_barrier() {
 
 __device__ __forceinline__ int lds_chunk(int row, int c) { return c ^ ((row >> 1) & 7); }
 
+// acc += a.b on v_mfma_i32_16x16x64_i8, accumulating in place in AGPRs. The
+// builtin lets the compiler pick another destination, and with all 256
+// accumulator registers taken it then copies tuples around in the K loop
+// (some 300 v_accvgpr moves per stage). The compiler knows neither that this
+// is an MFMA nor its wait states: accumulators written by other instructions
+// settle before the first one (acc_zero), and none is read before
+// acc_ready; the fragments come from LDS reads, whose waits it does count.
+__device__ __forceinline__ void mfma_tied(v4i& acc, const v4i& a, const v4i& b) {
+  __asm__("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+
+// Wait states between the accumulators' last MFMAs and their first other
+// use (at most 18 are needed), tied to the accumulators so that no read
+// moves above it.
+template <int NR>
+__device__ __forceinline__ void acc_ready(v4i (&acc)[NR][8]) {
+  __asm__ volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    __asm__ volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]),
+                          "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7]));
+}
+
+// The accumulators set to zero, and the wait states before an MFMA reads
+// them.
+template <int NR>
+__device__ __forceinline__ void acc_zero(v4i (&acc)[NR][8]) {
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = v4i{};
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+    __asm__ volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]),
+                          "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7]));
+  __asm__ volatile("s_nop 7" ::: "memory");
+}
+
 // f(integral_constant<int, I>) for I = LO .. HI - 1.
 template <int LO, int HI, typename F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -853,7 +859,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int EPI, int OUT, int FLAGS, int NB>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void gemm_i8_persistent(GemmParams p) {
-  // NB MFMA column blocks per wave. NB = 4 or 3: tiles are 256 x 64 NB
+  // NR = 2 NB MFMA column blocks per wave. NB = 4 or 3: tiles are 256 x 64 NB
   // (256 or 192 columns), the waves 2 x 2 quadrants of 128 x 32 NB. NB = 2:
   // tiles are 128 x 256 (for M of a few hundred rows), the waves 1 x 4
   // quadrants of 128 x 64 sharing the A tile, which fills half its slot. An
@@ -861,7 +867,7 @@ void gemm_i8_persistent(GemmParams p) {
   static_assert(NB == 4 || ((NB == 3 || NB == 2) && (FLAGS & kWithRope) == 0),
                 "NB 4, or 3 or 2 without the RoPE epilogue");
   constexpr int BM = NB == 2 ? 128 : 256, BN = NB == 2 ? 256 : 64 * NB, WN = 32 * NB;
-  constexpr int NA = BM / 32, JB = BN / 32;
+  constexpr int NA = BM / 32, JB = BN / 32, NR = 2 * NB;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -939,89 +945,80 @@ void gemm_i8_persistent(GemmParams p) {
     else dma16(p.a + (off_a[J] + kof), st);
     if constexpr (B && J == JB - 1) advance();
   };
-  // Part R (of NB, one per MFMA row) of half H of a unit: instructions
-  // [C H + R C / NB, C H + (R + 1) C / NB) with C the half's length.
-  auto dma_part = [&](auto b_tag, auto h_tag, auto r_tag, int base) {
-    constexpr bool B = decltype(b_tag)::value;
-    constexpr int H = decltype(h_tag)::value, R = decltype(r_tag)::value;
-    constexpr int C = B ? JB / 2 : NA / 2;
-    static_for<C * H + R * C / NB, C * H + (R + 1) * C / NB>([&](auto j) { dma_one(b_tag, j, base); });
-  };
-  auto issue_half = [&](auto b_tag, auto h_tag, int base) {
-    constexpr bool B = decltype(b_tag)::value;
-    constexpr int H = decltype(h_tag)::value, C = B ? JB / 2 : NA / 2;
-    static_for<C * H, C * H + C>([&](auto j) { dma_one(b_tag, j, base); });
+  auto issue_unit = [&](auto b_tag, int base) {
+    static_for<0, decltype(b_tag)::value ? JB : NA>([&](auto j) { dma_one(b_tag, j, base); });
   };
   using A_ = std::false_type;
   using B_ = std::true_type;
-  using H0 = std::integral_constant<int, 0>;
-  using H1 = std::integral_constant<int, 1>;
 
-  // v_mfma_i32_32x32x32_i8: for sub-step u (K bytes [32 u, 32 u + 32) of the
-  // stage), lane (r = lane % 32, h = lane / 32) supplies row r, logical
-  // chunk 2 u + h of both operands. Each wave holds a 4x4 grid of 32x32
-  // accumulator tiles (its 128x128 quadrant).
+  // v_mfma_i32_16x16x64_i8: for sub-step u (K bytes [64 u, 64 u + 64) of the
+  // stage), lane (r = lane % 16, h = lane / 16) supplies row r, logical
+  // chunk 4 u + h of both operands. Each wave holds an NR x 8 grid of 16x16
+  // accumulator tiles (its 128 x 32 NB quadrant).
   const int wm = NB == 2 ? 0 : wave >> 1, wn = NB == 2 ? wave : wave & 1;
-  const int fr = lane & 31, fh = lane >> 5;
+  const int fr = lane & 15, fh = lane >> 4;
   const int a_row = wm * 128 * kSK + fr * kSK, b_row = wn * WN * kSK + fr * kSK;
-  auto read_frags = [&](int base_a, int base_b, int u, v4i (&fa)[NB], v4i (&fb)[4]) {
-    const int8_t* sa = smem + base_a;
-    const int8_t* sb = smem + base_b;
-    const int off = lds_chunk(fr, 2 * u + fh) << 4;   // rows 32 i + fr share (row >> 1) & 7
-#pragma unroll
-    for (int i = 0; i < NB; ++i) fa[i] = *reinterpret_cast<const v4i*>(sb + b_row + i * 32 * kSK + off);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) fb[i] = *reinterpret_cast<const v4i*>(sa + a_row + i * 32 * kSK + off);
+  // Fragment read I of sub-step u, in the order its first MFMA row consumes
+  // them: the eight A fragments fb, then the B fragments fa.
+  constexpr int kReads = 8 + NR;
+  auto read_one = [&](int base_a, int base_b, int u, auto i_tag, v4i (&fa)[NR], v4i (&fb)[8]) {
+    constexpr int I = decltype(i_tag)::value;
+    const int off = lds_chunk(fr, 4 * u + fh) << 4;   // rows 16 i + fr share (row >> 1) & 7
+    if constexpr (I < 8) fb[I] = *reinterpret_cast<const v4i*>(smem + base_a + a_row + off + I * 16 * kSK);
+    else fa[I - 8] = *reinterpret_cast<const v4i*>(smem + base_b + b_row + off + (I - 8) * 16 * kSK);
   };
-  // Group k (0 .. NB - 2) of the fragment reads of sub-step u, in the order
-  // the next sub-step's first MFMA row consumes them (all four A fragments
-  // fb, then the B fragments fa). NB = 4: k = 0 reads fb[0..2], k = 1
-  // fb[3], fa[0..1], k = 2 fa[2..3]; NB = 3: k = 0 fb[0..3], k = 1
-  // fa[0..2]; NB = 2: k = 0 all six. The last MFMA row of a sub-step issues
-  // no reads, so the reads have landed when the next sub-step starts.
-  auto read_group = [&](int base_a, int base_b, int u, int k, v4i (&fa)[NB], v4i (&fb)[4]) {
-    const int off = lds_chunk(fr, 2 * u + fh) << 4;
-    const int8_t* sa = smem + base_a + a_row + off;
-    const int8_t* sb = smem + base_b + b_row + off;
-    auto rd = [](const int8_t* base, int i) { return *reinterpret_cast<const v4i*>(base + i * 32 * kSK); };
-    if constexpr (NB == 4) {
-      if (k == 0) {
-        fb[0] = rd(sa, 0); fb[1] = rd(sa, 1); fb[2] = rd(sa, 2);
-      } else if (k == 1) {
-        fb[3] = rd(sa, 3); fa[0] = rd(sb, 0); fa[1] = rd(sb, 1);
-      } else {
-        fa[2] = rd(sb, 2); fa[3] = rd(sb, 3);
-      }
-    } else if constexpr (NB == 3) {
-      if (k == 0) {
-        fb[0] = rd(sa, 0); fb[1] = rd(sa, 1); fb[2] = rd(sa, 2); fb[3] = rd(sa, 3);
-      } else {
-        fa[0] = rd(sb, 0); fa[1] = rd(sb, 1); fa[2] = rd(sb, 2);
-      }
-    } else {
-      fb[0] = rd(sa, 0); fb[1] = rd(sa, 1); fb[2] = rd(sa, 2); fb[3] = rd(sa, 3);
-      fa[0] = rd(sb, 0); fa[1] = rd(sb, 1);
-    }
+  auto read_frags = [&](int base_a, int base_b, int u, v4i (&fa)[NR], v4i (&fb)[8]) {
+    static_for<0, kReads>([&](auto i_tag) { read_one(base_a, base_b, u, i_tag, fa, fb); });
   };
-  v16i acc[NB][4];
-  // Block row nb of the NB x 4 MFMA grid (4 MFMAs).
-  auto mfma_row = [&](int nb, const v4i (&fa)[NB], const v4i (&fb)[4]) {
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-      acc[nb][mb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[nb], fb[mb], acc[nb][mb], 0, 0, 0);
+  v4i acc[NR][8];
+  // A sub-step: its 8 NR MFMAs (block T / 8, T % 8 of the grid in order),
+  // with the next sub-step's fragment reads and the C DMA instructions of a
+  // unit spread between them, one after an MFMA: an MFMA takes 16 cycles, in
+  // which the wave can issue one LDS read or DMA for free, but not a row's
+  // worth of them at once. The reads come after MFMAs T0 .. 8 NR - 9, so they
+  // have landed when the sub-step ends; at(T0) runs after MFMA T0 - 1.
+  auto substep = [&](const v4i (&ca)[NR], const v4i (&cb)[8], auto t0_tag, auto&& at_t0, int ra, int rb, int u,
+                     v4i (&na)[NR], v4i (&nb)[8], auto b_tag, int dbase) {
+    constexpr int T0 = decltype(t0_tag)::value, L = 8 * (NR - 1) - T0;
+    constexpr int C = decltype(b_tag)::value ? JB : NA, D = 8 * NR - T0;
+    static_for<0, 8 * NR>([&](auto t_tag) {
+      constexpr int T = decltype(t_tag)::value;
+      if constexpr (T0 > 0 && T == T0) at_t0();
+      mfma_tied(acc[T / 8][T % 8], ca[T / 8], cb[T % 8]);
+      if constexpr (T >= T0) {
+        constexpr int S = T - T0;
+        // Reads i with floor(i L / kReads) == S and DMA j with floor(j D / C) + 1 == S.
+        static_for<(S * kReads + L - 1) / L, ((S + 1) * kReads + L - 1) / L>([&](auto i_tag) {
+          if constexpr (decltype(i_tag)::value < kReads) {
+            __builtin_amdgcn_sched_barrier(0);
+            read_one(ra, rb, u, i_tag, na, nb);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        });
+        if constexpr (S >= 1)
+          static_for<((S - 1) * C + D - 1) / D, (S * C + D - 1) / D>([&](auto j_tag) {
+            __builtin_amdgcn_sched_barrier(0);
+            dma_one(b_tag, j_tag, dbase);
+            __builtin_amdgcn_sched_barrier(0);
+          });
+      }
+    });
   };
 
   // Stage g computes from units 2g, 2g + 1 (slots c, c + 1 with
-  // c = 2g mod 5). During it the second half of unit 2g + 3 and unit 2g + 4
-  // are issued (slots c + 3, c + 4, freed by stage g - 1); its end releases
-  // slots c, c + 1, and the first half of unit 2g + 5 goes to slot c.
+  // c = 2g mod 5). Its first sub-step issues unit 2g + 4 (slot c + 4, freed
+  // by stage g - 1); the barrier after the second sub-step's first MFMA row
+  // releases slots c, c + 1 (that row has consumed the stage's last
+  // fragments), and unit 2g + 5 then goes to slot c.
   //
   // 128 x 256 tiles (NB = 2) take a ring of three whole stages instead
   // (STAGE_RING): stage slot s holds the A tile (16 KB) at 48 KB s and the
-  // B tile (32 KB) after it. Stage g computes from slot g mod 3 while stage
-  // g + 1 (issued during stage g - 1) lands and stage g + 2 is issued into
-  // the slot stage g - 1 released: two stages (96 KB) in flight, where the
-  // five half-stage slots keep about one (their A slots half empty).
+  // B tile (32 KB) after it. Stage g computes from slot g mod 3; its first
+  // sub-step issues the B tile of stage g + 2 into the slot stage g - 1
+  // released (the A tile went there after that release), and after its own
+  // barrier it issues the A tile of stage g + 3 into its own slot: two stages
+  // (96 KB) in flight, where the five half-stage slots keep about one (their
+  // A slots half empty).
   constexpr bool STAGE_RING = NB == 2;
   constexpr int kStage2 = (BM + BN) * kSK, kA2 = BM * kSK;
   static_assert(!STAGE_RING || 3 * kStage2 <= kPersistentLds, "three stages fit the LDS");
@@ -1030,28 +1027,18 @@ void gemm_i8_persistent(GemmParams p) {
   // or whose A tile is in slot s (its B tile in the next slot).
   auto a_of = [&](int s) { return STAGE_RING ? s * kStage2 : s * kSTile; };
   auto b_of = [&](int s) { return STAGE_RING ? s * kStage2 + kA2 : next_slot(s) * kSTile; };
+  issue_unit(A_{}, a_of(0));
+  issue_unit(B_{}, b_of(0));
+  issue_unit(A_{}, a_of(STAGE_RING ? 1 : 2));
+  issue_unit(B_{}, b_of(STAGE_RING ? 1 : 2));
   if constexpr (STAGE_RING) {
-    issue_half(A_{}, H0{}, a_of(0));
-    issue_half(A_{}, H1{}, a_of(0));
-    issue_half(B_{}, H0{}, b_of(0));
-    issue_half(B_{}, H1{}, b_of(0));
-    issue_half(A_{}, H0{}, a_of(1));
-    issue_half(A_{}, H1{}, a_of(1));
-    issue_half(B_{}, H0{}, b_of(1));
-    issue_half(B_{}, H1{}, b_of(1));
-    wait_vmcnt<NA + JB>();  // stage 0 landed (stage 1 in flight)
+    issue_unit(A_{}, a_of(2));
+    wait_vmcnt<2 * NA + JB>();  // stage 0 landed
   } else {
-    issue_half(A_{}, H0{}, 0);
-    issue_half(A_{}, H1{}, 0);
-    issue_half(B_{}, H0{}, kSTile);
-    issue_half(B_{}, H1{}, kSTile);
-    issue_half(A_{}, H0{}, 2 * kSTile);
-    issue_half(A_{}, H1{}, 2 * kSTile);
-    issue_half(B_{}, H0{}, 3 * kSTile);
-    wait_vmcnt<NA + JB / 2>();  // stage 0 landed (unit 2 and half of unit 3 in flight)
+    wait_vmcnt<NA + JB>();
   }
   block_barrier();
-  v4i fa0[NB], fb0[4], fa1[NB], fb1[4];
+  v4i fa0[NR], fb0[8], fa1[NR], fb1[8];
   read_frags(a_of(0), b_of(0), 0, fa0, fb0);
   int cur_a = 0;   // slot of the current stage (STAGE_RING) or of its A tile
   for (int i = 0; i < ntiles; ++i) {
@@ -1059,16 +1046,17 @@ void gemm_i8_persistent(GemmParams p) {
     int tm, tn;
     raster(item / ksplit, tiles_m, tiles_n, tm, tn);
     const int mw = tm * BM + wm * 128, nw = tn * BN + wn * WN;
-    // Row scales in the MFMA layout, the column scales (and biases) of the
-    // staged read-out and the gate labels, fetched before the K loop so the
+    // Row scales (lane % 32's row of each 32-row block), the column scales
+    // (and biases) of the staged read-out and the gate labels, fetched before the K loop so the
     // epilogue never waits on them.
     float as[4], wsc[2][8];
     uint32_t braw[2][8];
     int lbl[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
-      as[mb] = EPI != kEpiInt32 ? p.row_scale[min(mw + mb * 32 + fr, p.m - 1)] : 0.0f;
-      if constexpr ((FLAGS & kWithGate) != 0) lbl[mb] = p.labels[min(mw + mb * 32 + fr, p.m - 1)];
+      const int m = min(mw + mb * 32 + (lane & 31), p.m - 1);
+      as[mb] = EPI != kEpiInt32 ? p.row_scale[m] : 0.0f;
+      if constexpr ((FLAGS & kWithGate) != 0) lbl[mb] = p.labels[m];
     }
     if constexpr ((FLAGS & kWithRope) != 0) {
 #pragma unroll
@@ -1080,99 +1068,40 @@ void gemm_i8_persistent(GemmParams p) {
     } else {
       load_readout_scales<EPI, OUT, (FLAGS & kWithBias) != 0>(p, nw, lane, wsc, braw);
     }
-#pragma unroll
-    for (int a = 0; a < NB; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = v16i{};
+    acc_zero(acc);
     const int nks = ks_end(item) - ks_begin(item);   // >= 1
-    // One stage: 16 NB MFMAs, 4 (NB + 4) fragment reads and NA + JB DMA
+    // One stage: 16 NR MFMAs, 2 (NR + 8) fragment reads and NA + JB DMA
     // instructions.
     int stg = 0;   // byte offset of the last stage's B tile: the epilogue's staging area
     int ks = 0;
-    // A sub-step in fixed order: each MFMA row of the current fragments but
-    // the last is followed by one group of the next sub-step's fragment
-    // reads, and every row by its part of the half-unit of DMA
-    // (sched_barrier keeps the compiler from regrouping them).
-    auto substep = [&](const v4i (&ca)[NB], const v4i (&cb)[4], int ra, int rb, int u, v4i (&na)[NB],
-                       v4i (&nb)[4], auto b_tag, auto h_tag, int dbase) {
-      static_for<0, NB>([&](auto r_tag) {
-        constexpr int R = decltype(r_tag)::value;
-        mfma_row(R, ca, cb);
-        // (The last row's DMA may rise among its MFMAs.)
-        if constexpr (R + 1 < NB) {
-          __builtin_amdgcn_sched_barrier(0);
-          read_group(ra, rb, u, R, na, nb);
-        }
-        dma_part(b_tag, h_tag, r_tag, dbase);
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    };
     do {  // nks >= 1
-      // At a tile's last stage the next tile's first fragments are read
-      // after the epilogue, so they do not hold registers through it.
-      const bool last = ks + 1 == nks;
-      if constexpr (STAGE_RING) {
-        // Stage g + 2 goes to the slot stage g - 1 released: its A tile
-        // during sub-steps 0 and 1, its B tile during 2 and 3.
-        using R0 = std::integral_constant<int, 0>;
-        using R1 = std::integral_constant<int, 1>;
-        const int nxt = next_slot(cur_a), fill = next_slot(nxt);
-        const int ca = a_of(cur_a), cb = b_of(cur_a);
-        substep(fa0, fb0, ca, cb, 1, fa1, fb1, A_{}, H0{}, a_of(fill));
-        substep(fa1, fb1, ca, cb, 2, fa0, fb0, A_{}, H1{}, a_of(fill));
-        substep(fa0, fb0, ca, cb, 3, fa1, fb1, B_{}, H0{}, b_of(fill));
-        mfma_row(0, fa1, fb1);
+      // Slot of the next stage (its A tile), and the tile the first sub-step
+      // fills: the B tile of stage g + 2 (STAGE_RING) or unit 2g + 4.
+      const int nxt = STAGE_RING ? next_slot(cur_a) : next_slot(next_slot(cur_a));
+      const int fill = STAGE_RING ? next_slot(nxt) : next_slot(next_slot(nxt));
+      const int ca = a_of(cur_a), cb = b_of(cur_a);
+      using First = std::conditional_t<STAGE_RING, B_, A_>;
+      using Second = std::conditional_t<STAGE_RING, A_, B_>;
+      const int fill_first = STAGE_RING ? b_of(fill) : a_of(fill);
+      using T0 = std::integral_constant<int, 0>;
+      using T8 = std::integral_constant<int, 8>;
+      substep(fa0, fb0, T0{}, [] {}, ca, cb, 1, fa1, fb1, First{}, fill_first);
+      substep(fa1, fb1, T8{}, [&] {
+        // The first row consumed the stage's last fragments. The next stage
+        // landed - only unit 2g + 4 (STAGE_RING: the A and B tiles of stage
+        // g + 2), issued after it, may still be in flight;
         __builtin_amdgcn_sched_barrier(0);
-        dma_part(B_{}, H1{}, R0{}, b_of(fill));
-        __builtin_amdgcn_sched_barrier(0);
-        // Stage g + 1 landed - only the NA + 3 JB / 4 instructions of stage
-        // g + 2 issued so far are younger - and this wave's reads of stage g
-        // returned; the barrier releases slot g mod 3 for stage g + 3.
-        wait_vm_lgkm<NA + 3 * JB / 4>();
-        block_barrier();
-        if (!last) read_group(a_of(nxt), b_of(nxt), 0, 0, fa0, fb0);
-        dma_part(B_{}, H1{}, R1{}, b_of(fill));
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_row(1, fa1, fb1);
-        __builtin_amdgcn_sched_barrier(0);
-        stg = cb;
-        cur_a = nxt;
-      } else {
-        const int cur_b = next_slot(cur_a);
-        const int nxt_a = next_slot(cur_b), nxt_b = next_slot(nxt_a), fill = next_slot(nxt_b);
-        substep(fa0, fb0, a_of(cur_a), a_of(cur_b), 1, fa1, fb1, B_{}, H1{}, a_of(nxt_b));
-        substep(fa1, fb1, a_of(cur_a), a_of(cur_b), 2, fa0, fb0, A_{}, H0{}, a_of(fill));
-        substep(fa0, fb0, a_of(cur_a), a_of(cur_b), 3, fa1, fb1, A_{}, H1{}, a_of(fill));
-        // The first MFMA row of the last sub-step consumes its fragments, so
-        // past it this wave is done reading the stage's slots.
-        mfma_row(0, fa1, fb1);
-        __builtin_amdgcn_sched_barrier(0);
-        // The next stage (units 2g + 2, 2g + 3) landed - only unit 2g + 4,
-        // issued after them, may still be in flight - and this wave's reads of
-        // this stage returned;
-        wait_vm_lgkm<NA>();
-        block_barrier();   // ... for every wave: both slots are released.
-        static_for<0, NB>([&](auto r_tag) {
-          constexpr int R = decltype(r_tag)::value;
-          if constexpr (R > 0) {
-            mfma_row(R, fa1, fb1);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-          if constexpr (R + 1 < NB) {
-            if (!last) read_group(a_of(nxt_a), a_of(nxt_b), 0, R, fa0, fb0);
-          }
-          dma_part(B_{}, H0{}, r_tag, a_of(cur_a));
-          __builtin_amdgcn_sched_barrier(0);
-        });
-        stg = a_of(cur_b);
-        cur_a = nxt_a;
-      }
+        wait_vm_lgkm<STAGE_RING ? NA + JB : NA>();
+        block_barrier();   // ... for every wave: the stage's slots are released.
+      }, a_of(nxt), b_of(nxt), 0, fa0, fb0, Second{}, ca);
+      stg = cb;
+      cur_a = nxt;
     } while (++ks < nks);
+    acc_ready(acc);
     // The tile's scale and bias loads have landed: they are older than the
-    // DMA still in flight (half-stage slots: at most unit 2g + 4 and the
-    // first half of unit 2g + 5; STAGE_RING: stage g + 2). (The epilogue's
-    // residual loads queue behind those instructions.)
-    wait_vmcnt<STAGE_RING ? NA + JB : NA + JB / 2>();
+    // two units of DMA its last stage issued. (The epilogue's residual loads
+    // queue behind those instructions.)
+    wait_vmcnt<NA + JB>();
     float bsc[2][8];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -1181,6 +1110,11 @@ void gemm_i8_persistent(GemmParams p) {
         bsc[h][j] = (FLAGS & kWithBias) == 0       ? 0.0f
                     : p.bias_dtype == kF16 ? h2f((uint16_t)braw[h][j])
                                            : __builtin_bit_cast(float, braw[h][j]);
+    // The epilogue's lane arithmetic starts from an opaque copy of the lane, so
+    // none of it is hoisted out of the tile loop to hold registers through
+    // the K loop, which needs them for its fragments.
+    int elane = lane;
+    __asm__ volatile("" : "+v"(elane));
     int8_t* const stage_w = smem + stg + wave * 8192;
     const int64_t out_off = (item % ksplit) * p.split_stride;
     // Interior quadrants take a copy without store masks (not for the gate
@@ -1188,31 +1122,31 @@ void gemm_i8_persistent(GemmParams p) {
     if constexpr ((FLAGS & kWithRope) != 0) {
       if (nw >= 2 * p.rope_heads * 128) {   // V columns
         if (p.vec16 && mw + 128 <= p.m && nw + 128 <= p.n)
-          store_quadrant32_passes<EPI, OUT, 0, true>(p, acc, wsc, bsc, as, lbl, mw, nw, lane, stage_w, out_off);
+          store_quadrant32_passes<EPI, OUT, 0, true>(p, acc, wsc, bsc, as, lbl, mw, nw, elane, stage_w, out_off);
         else
-          store_quadrant32_passes<EPI, OUT, 0, false>(p, acc, wsc, bsc, as, lbl, mw, nw, lane, stage_w, out_off);
+          store_quadrant32_passes<EPI, OUT, 0, false>(p, acc, wsc, bsc, as, lbl, mw, nw, elane, stage_w, out_off);
       } else if (p.rope_pairs) {
-        if (p.rope_f32) store_quadrant_rope<EPI, kF32, true>(p, acc, wsc, as, mw, nw, lane, stage_w);
-        else store_quadrant_rope<EPI, kF16, true>(p, acc, wsc, as, mw, nw, lane, stage_w);
+        if (p.rope_f32) store_quadrant_rope<EPI, kF32, true>(p, acc, wsc, as, mw, nw, elane, stage_w);
+        else store_quadrant_rope<EPI, kF16, true>(p, acc, wsc, as, mw, nw, elane, stage_w);
       } else if (p.rope_f32) {
-        store_quadrant_rope<EPI, kF32, false>(p, acc, wsc, as, mw, nw, lane, stage_w);
+        store_quadrant_rope<EPI, kF32, false>(p, acc, wsc, as, mw, nw, elane, stage_w);
       } else {
-        store_quadrant_rope<EPI, kF16, false>(p, acc, wsc, as, mw, nw, lane, stage_w);
+        store_quadrant_rope<EPI, kF16, false>(p, acc, wsc, as, mw, nw, elane, stage_w);
       }
     } else if ((FLAGS & kWithGate) == 0 && p.vec16 && mw + 128 <= p.m && nw + WN <= p.n)
       store_quadrant32_passes<EPI, OUT, FLAGS, (FLAGS & kWithGate) == 0, NB>(p, acc, wsc, bsc, as, lbl, mw, nw,
-                                                                            lane, stage_w, out_off);
+                                                                            elane, stage_w, out_off);
     else
-      store_quadrant32_passes<EPI, OUT, FLAGS, false, NB>(p, acc, wsc, bsc, as, lbl, mw, nw, lane, stage_w,
+      store_quadrant32_passes<EPI, OUT, FLAGS, false, NB>(p, acc, wsc, bsc, as, lbl, mw, nw, elane, stage_w,
                                                           out_off);
-    // The staging slot's next unit (2g + 6; STAGE_RING: the B tile of stage
+    // The staging tile's next unit (2g + 6; STAGE_RING: the B tile of stage
     // g + 3) is issued during the next stage; a wave's DMA into a slot
     // writes the same 8 KB it used for staging, so its own staging reads
     // returning is all that unit waits for.
     wait_lgkm();
-    // The next tile's first fragments (its stage 0 landed before the last
-    // barrier).
-    static_for<0, NB - 1>([&](auto k) { read_group(a_of(cur_a), b_of(cur_a), 0, decltype(k)::value, fa0, fb0); });
+    // The next tile's first fragments, read again (the last stage read them
+    // too, but they would hold registers through the epilogue).
+    read_frags(a_of(cur_a), b_of(cur_a), 0, fa0, fb0);
   }
   wait_vmcnt<0>();  // no DMA may still target this workgroup's LDS at exit
 }

@@ -75,6 +75,23 @@ def test_gemm_dispatch_sweep(gpu, m, n, k):
         assert_bits_equal(np_of(got), want, f'row f16 {m}x{n}x{k} ws={workspace is None}')
 
 
+@pytest.mark.parametrize('m,n', [(4300, 4200), (6814, 5376), (353, 25000)])
+@pytest.mark.parametrize('k', [128, 256, 384, 1152, 3584])
+def test_gemm_stage_ring_across_tiles(gpu, m, n, k):
+    """More output tiles of each tile shape than CUs at 1, 2, 3, 9 and 28
+    stages: the operand ring crosses tile boundaries at every phase. int32
+    sums are exact in float64 (|C| <= 3584 * 2^14 < 2^53)."""
+    g = torch.Generator(device=gpu).manual_seed(m + n + k)
+    a = torch.randint(-128, 128, (m, k), generator=g, device=gpu, dtype=torch.int8)
+    b = torch.randint(-128, 128, (n, k), generator=g, device=gpu, dtype=torch.int8)
+    want = (a.double() @ b.double().t().contiguous()).to(torch.int32)
+    assert torch.equal(kernels.gemm(a, b), want)
+    rs = torch.rand((m, 1), generator=g, device=gpu) * 0.01 + 1e-4
+    ws = torch.rand((n, 1), generator=g, device=gpu) * 1e-3 + 1e-6
+    got = kernels.gemm(a, b, epilogue=kernels.EPI_ROW, row_scale=rs, col_scale=ws, out_dtype=torch.float16)
+    assert torch.equal(got, ((want.float() * rs) * ws.t()).half())
+
+
 def test_gemm_signed_extremes_and_layout(gpu):
     k = 5120
     a = torch.full((33, k), -128, dtype=torch.int8)
