@@ -176,3 +176,54 @@ def test_strided_operands_and_output(gpu, b, h, n, dtype):
     kernels.attention_prepare(odd, odd, odd)
     with pytest.raises(ValueError):
         kernels.attention(flat, out_dtype=torch.float32, out=torch.empty((b, h, n, 130), device=gpu)[..., :128])
+
+
+# The preparation's own edges: chunks of 256 keys and their batches of 32
+# (remainders), fp32's two phases to a chunk, 32 chunks (the last count the
+# quantizer reduces itself) and 33 (the finishing kernel).
+@pytest.mark.parametrize('nq,nk,dtype', [(5, 31, torch.float32), (130, 33, torch.float16), (1, 255, torch.float32),
+                                         (128, 256, torch.float16), (129, 257, torch.float32), (3, 385, torch.float32),
+                                         (2, 8192, torch.float16), (2, 8193, torch.float32)])
+def test_prepare_chunk_edges(gpu, nq, nk, dtype):
+    g = torch.Generator().manual_seed(nq + 31 * nk)
+    q, k, v = _qkv(g, 1, 2, nq, nk, dtype)
+    prep = kernels.attention_prepare(q.to(gpu), k.to(gpu), v.to(gpu))
+    want = oa.gpu_operands(oa.kitchen_prepare(_np(q), _np(k), _np(v), cta_k=oa.GPU_CTA_K))
+    for name in oa.GPU_OPERANDS:
+        assert np_of(prep[name]).tobytes() == np.ascontiguousarray(want[name]).tobytes(), name
+
+
+def test_prepare_ties_and_wide_scales(gpu):
+    """Codes where x / s lies on or next to a tie (the reciprocal product does
+    not decide), and scales whose reciprocal is not a normal number."""
+    g = torch.Generator().manual_seed(77)
+    half = torch.randint(-254, 255, (1, 3, 140, 128), generator=g).float() * 0.5
+    half[..., 0] = 127.0
+    q, k, v = half.clone(), half - half.mean(2, keepdim=True), half.clone()
+    q[:, 1] *= 3e38 / 127.0
+    v[:, 1] *= 3e38 / 127.0
+    q[:, 2] *= 1e-38
+    v[:, 2] *= 1e-38
+    prep = kernels.attention_prepare(q.to(gpu), k.to(gpu), v.to(gpu))
+    want = oa.gpu_operands(oa.kitchen_prepare(_np(q), _np(k), _np(v), cta_k=oa.GPU_CTA_K))
+    for name in oa.GPU_OPERANDS:
+        assert np_of(prep[name]).tobytes() == np.ascontiguousarray(want[name]).tobytes(), name
+
+
+@pytest.mark.parametrize('nq,nk', [(33, 1600), (64, 1664), (40, 1792), (33, 1920), (32, 130), (200, 64)])
+def test_both_kernels_match_oracle(gpu, nq, nk):
+    """260 heads fill the GPU with 128-query workgroups; one head alone takes
+    the kernel that splits the keys over a workgroup's waves. Both follow the
+    oracle, at every tail of the step loop (one to three waves without a last
+    block, a single block)."""
+    g = torch.Generator().manual_seed(nq + nk)
+    q, k, v = _qkv(g, 1, 260, nq, nk, torch.float16)
+    many = np_of(kernels.attention(kernels.attention_prepare(q.to(gpu), k.to(gpu), v.to(gpu)), out_dtype=torch.float32))
+    for h in (0, 259):
+        qh, kh, vh = (t[:, h:h + 1].contiguous() for t in (q, k, v))
+        one = np_of(kernels.attention(kernels.attention_prepare(qh.to(gpu), kh.to(gpu), vh.to(gpu)),
+                                      out_dtype=torch.float32))
+        want = oa.kitchen_attention(oa.kitchen_prepare(_np(qh), _np(kh), _np(vh), cta_k=oa.GPU_CTA_K))
+        # 1e-5: the bound of test_attention_matches_oracle (hardware exp2, FP32 order)
+        for out in (many[:, h:h + 1], one):
+            assert np.abs(out - want).max() <= 1e-5 * np.abs(want).max()
