@@ -485,6 +485,18 @@ typedef struct W8A8DequantArgs {
 
 int w8a8_dequantize(const W8A8DequantArgs* args);
 
+/*
+ * Modulation labels: labels[r] = values[i] for the rows r of segment i, which
+ * are [ends[i - 1], ends[i]) with ends[-1] = 0.
+ * Replaces: patches/tilelang_dit_fusion.py:106-124 (labels built per
+ *           forward and copied to the device).
+ * ends, values: HOST arrays of count entries, read before the call returns;
+ *   ends strictly ascending with ends[count - 1] == rows.
+ * labels: device int32 [rows].
+ */
+int w8a8_segment_labels(const int32_t* ends, const int32_t* values, int64_t count, int32_t* labels, int64_t rows,
+                        void* stream);
+
 /* ABI version (W8A8_ABI_VERSION). */
 int w8a8_abi_version(void);
 

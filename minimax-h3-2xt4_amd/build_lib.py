@@ -1,4 +1,5 @@
-"""Compile the gfx950 HIP sources into the in-tree C-ABI library libw8a8.so.
+"""Compile the gfx950 HIP sources into the in-tree C-ABI library libw8a8.so,
+and csrc/native.cpp (host C++ on torch's tensors) into the module _native.
 
     python minimax-h3-2xt4_amd/build_lib.py [--jobs N] [--verbose]
 
@@ -13,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -20,6 +22,7 @@ ROOT = PKG.parent
 CSRC = PKG / 'csrc'
 BUILD = PKG / '_build'
 OUT = PKG / 'w8a8' / 'libw8a8.so'
+NATIVE_OUT = PKG / 'w8a8' / '_native.so'
 ARCH = 'gfx950'
 
 HIPCC_FLAGS = [
@@ -78,12 +81,45 @@ def _compile(unit, verbose):
     return obj
 
 
+def _run(cmd, what, verbose):
+    if verbose:
+        print(' '.join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f'{what} failed:\n{res.stdout}\n{res.stderr}')
+
+
+def _compile_native(verbose):
+    """Object of csrc/native.cpp: plain host C++ against torch's headers."""
+    from torch.utils.cpp_extension import include_paths
+    import torch
+    obj = BUILD / 'native.o'
+    rocm = Path(hipcc()).resolve().parents[1]
+    _run(['g++', '-O2', '-std=c++17', '-fPIC', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+          f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}', f'-I{ROOT / "include"}',
+          *(f'-isystem{p}' for p in include_paths()), f'-isystem{rocm / "include"}',
+          f'-isystem{sysconfig.get_paths()["include"]}', '-c', str(CSRC / 'native.cpp'), '-o', str(obj)],
+         'g++ native.cpp', verbose)
+    return obj
+
+
+def _link_native(obj, verbose):
+    from torch.utils.cpp_extension import library_paths
+    tmp = NATIVE_OUT.with_suffix('.so.tmp')
+    _run(['g++', '-shared', '-fPIC', str(obj), '-o', str(tmp), f'-L{OUT.parent}', '-l:libw8a8.so', '-Wl,-rpath,$ORIGIN',
+          *(f'-L{p}' for p in library_paths()), '-ltorch_python', '-ltorch_cpu', '-lc10', '-lc10_hip'],
+         'link _native', verbose)
+    os.replace(tmp, NATIVE_OUT)
+
+
 def build(jobs=None, verbose=False):
     BUILD.mkdir(exist_ok=True)
     units = _units()
-    jobs = jobs or min(len(units), max(1, os.cpu_count() or 4))
+    jobs = jobs or min(len(units) + 1, max(1, os.cpu_count() or 4))
     with cf.ThreadPoolExecutor(max_workers=jobs) as pool:
+        native = pool.submit(_compile_native, verbose)
         objs = list(pool.map(lambda u: _compile(u, verbose), units))
+        native = native.result()
     tmp = OUT.with_suffix('.so.tmp')
     cmd = [hipcc(), f'--offload-arch={ARCH}', '-shared', '-fPIC', *map(str, objs), '-o', str(tmp)]
     if verbose:
@@ -92,6 +128,7 @@ def build(jobs=None, verbose=False):
     if res.returncode != 0:
         raise RuntimeError(f'link failed:\n{res.stdout}\n{res.stderr}')
     os.replace(tmp, OUT)
+    _link_native(native, verbose)
     return OUT
 
 

@@ -95,10 +95,11 @@ STRUCT_ENTRY_POINTS = ('w8a8_quantize_rows', 'w8a8_swiglu_quantize', 'w8a8_gemm'
                        'w8a8_norm_quantize', 'w8a8_rms_rope', 'w8a8_attention_prepare', 'w8a8_attention')
 ENTRY_POINTS = STRUCT_ENTRY_POINTS + ('w8a8_gemm_noalloc', 'w8a8_abi_version', 'w8a8_struct_size',
                                       'w8a8_last_error', 'w8a8_gemm_workspace_size',
-                                      'w8a8_attention_workspace_size')
+                                      'w8a8_attention_workspace_size', 'w8a8_segment_labels')
 GEMM_SCRATCH_BYTES = 64 << 20   # W8A8_GEMM_SCRATCH_BYTES: the no-allocation GEMM's split-K scratch per GPU
 
 _LIB = None
+_NATIVE = None
 
 
 class W8A8Error(RuntimeError):
@@ -127,6 +128,8 @@ def load(path=None):
     lib.w8a8_gemm_workspace_size.argtypes = [_c.c_int64, _c.c_int64, _c.c_int64]
     lib.w8a8_attention_workspace_size.restype = _c.c_int64
     lib.w8a8_attention_workspace_size.argtypes = [_c.c_int64, _c.c_int64, _c.c_int64]
+    lib.w8a8_segment_labels.restype = _c.c_int
+    lib.w8a8_segment_labels.argtypes = [_p, _p, _c.c_int64, _p, _c.c_int64, _p]
     for name, st in zip(STRUCT_ENTRY_POINTS + ('w8a8_gemm_noalloc',), STRUCTS + (GemmArgs,)):
         fn = getattr(lib, name)
         fn.restype = _c.c_int
@@ -140,6 +143,18 @@ def load(path=None):
     if path is None:
         _LIB = lib
     return lib
+
+
+def native():
+    """The module of the host-bound calls (csrc/native.cpp), linked to the
+    library; loaded on first use, and like it without a fallback."""
+    global _NATIVE
+    if _NATIVE is None:
+        load()
+        from . import _native
+        _native.set_error_class(W8A8Error)
+        _NATIVE = _native
+    return _NATIVE
 
 
 def call(name, args):

@@ -7,7 +7,7 @@ fp16(f32(C) * (a * w)) so no int32 accumulator reaches HBM.
 """
 import torch
 
-from . import kernels
+from . import _abi, kernels
 
 _BACKENDS = ('preallocated', 'cuda_int8_tilelang')
 
@@ -66,6 +66,10 @@ def column_linear(x, weight, weight_scale, *, convrot=True, convrot_groupsize=25
         raise ValueError('Unknown column linear backend')
     if x.shape[-1] != weight.shape[-1]:
         raise ValueError('Input and weight inner dimensions must match')
+    if convrot and convrot_groupsize == 256:
+        output = _abi.native().linear(x, weight, weight_scale, bias, _abi.EPI_COLUMN, 1, out_dtype)
+        if output is not None:
+            return output
     shape = x.shape
     weight = weight.to(device=x.device).contiguous()
     scale = _weight_scale(weight, weight_scale, x.device)

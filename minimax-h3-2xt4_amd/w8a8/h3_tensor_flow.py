@@ -17,7 +17,7 @@ from dataclasses import dataclass
 import torch
 from torch import nn
 
-from . import kernels
+from . import _abi, kernels
 
 
 @dataclass(frozen=True)
@@ -155,7 +155,13 @@ def segment_key(rows, segments, modulation_rows=9):
 
 def labels_for(rows, segments, modulation_rows=9, device=None):
     """int32 [rows] gate-table row of every row, or None when the segments do
-    not tile the rows (patches/tilelang_dit_fusion.py:106-124)."""
+    not tile the rows (patches/tilelang_dit_fusion.py:106-124). On the current
+    GPU a kernel writes them (no copy from the host, which would wait for the
+    stream)."""
+    if isinstance(device, torch.device) and device.type == 'cuda' and device.index is not None:
+        labels = _abi.native().segment_labels(rows, segments, modulation_rows, device.index)
+        if labels is not None:
+            return labels
     key = segment_key(rows, segments, modulation_rows)
     if key is None:
         return None

@@ -16,7 +16,7 @@ from dataclasses import dataclass
 
 import torch
 
-from . import kernels
+from . import _abi, kernels
 
 
 @dataclass
@@ -45,4 +45,8 @@ def int8_attention_from_prequantized(prepared):
 
 def int8_attention(q, k, v, *, scale=None, attn_mask=None):
     """patches/kitchen_attention.py:227-238: attention of [B, H, N, 128] q, k, v."""
+    if attn_mask is None:
+        out = _abi.native().int8_attention(q, k, v, scale)
+        if out is not None:
+            return out
     return int8_attention_from_prequantized(prequantize_int8_attention(q, k, v, scale=scale, attn_mask=attn_mask))

@@ -7,7 +7,7 @@ exchange are identities on one rank).
 """
 import torch
 
-from . import kernels
+from . import _abi, kernels
 
 GROUPSIZE = 256
 
@@ -71,6 +71,10 @@ def row_linear(x, weight, weight_scale, comm, world_size, groupsize=GROUPSIZE, i
     addcmul(residual, out, residual_scale) after the storage cast.
     """
     _single_rank(world_size)
+    if input_act is None and residual is None and groupsize == GROUPSIZE:
+        out = _abi.native().linear(x, weight, weight_scale, bias, _abi.EPI_ROW, 0, x.dtype)
+        if out is not None:
+            return out
     q, scale = quantize(x, groupsize, input_act=input_act)
     out_dtype = x.dtype if x.dtype in (torch.float16, torch.bfloat16, torch.float32) else torch.float32
     out = kernels.gemm(q, weight, epilogue=kernels.EPI_ROW, row_scale=scale, col_scale=weight_scale, bias=bias,

@@ -223,3 +223,22 @@ def test_empty_problems_return_ok_without_launch():
 def test_missing_library_fails_loudly(tmp_path):
     with pytest.raises(RuntimeError, match='no CPU fallback'):
         _abi.load(tmp_path / 'libw8a8.so')
+
+
+def test_segment_labels_checks():
+    lib = _abi.load()
+
+    def call(ends, values, rows, labels=4096):
+        n = len(ends)
+        rc = lib.w8a8_segment_labels((ctypes.c_int32 * n)(*ends), (ctypes.c_int32 * n)(*values), n, labels, rows, None)
+        return rc, lib.w8a8_last_error().decode()
+
+    for ends in ([3, 3, 8], [5, 4, 8], [0, 8], [9]):
+        rc, msg = call(ends, [0] * len(ends), 8)
+        assert rc == _abi.ERR_INVALID and 'ascend' in msg, ends
+    rc, msg = call([4, 7], [0, 1], 8)
+    assert rc == _abi.ERR_INVALID and 'cover' in msg
+    rc, msg = call([], [], 8)
+    assert rc == _abi.ERR_INVALID
+    rc, msg = call([8], [0], 8, labels=None)
+    assert rc == _abi.ERR_INVALID and 'null' in msg

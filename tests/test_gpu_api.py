@@ -265,3 +265,59 @@ def test_row_linear_writes_into_a_row_range(gpu):
     assert got.data_ptr() == full[20:90].data_ptr()
     assert torch.equal(full[20:90], want)
     assert torch.isnan(full[:20]).all() and torch.isnan(full[90:]).all()
+
+
+@pytest.mark.parametrize('count', [1, 16, 128, 129, 300])
+def test_segment_labels_on_device(gpu, count):
+    """The labels kernel (up to 128 segments a launch) against the host's."""
+    from w8a8.h3_tensor_flow import labels_for
+    for rows in (count, 3 * count + 5, 53504):
+        bounds = [rows * i // count for i in range(count + 1)]
+        segs = [(a, b, (7 * i) % 9) for i, (a, b) in enumerate(zip(bounds, bounds[1:]))]
+        segs = segs[::-1]
+        got = labels_for(rows, segs, 9, device=torch.device('cuda', torch.cuda.current_device()))
+        assert got.dtype == torch.int32 and got.is_cuda
+        assert torch.equal(got.cpu(), labels_for(rows, segs, 9))
+        assert labels_for(rows + 1, segs, 9, device=gpu) is None
+
+
+@pytest.mark.parametrize('m,dtype,bias', [(1, torch.float16, None), (1, torch.bfloat16, torch.float32),
+                                          (5, torch.float32, torch.float16), (70, torch.float16, torch.float16)])
+def test_native_linear_equals_two_calls(gpu, m, dtype, bias):
+    """The native call of a plain projection gives the bits of the quantizer
+    and the GEMM called one by one, and leaves other layouts (a longer row
+    stride) to the Python route, which does too."""
+    from w8a8 import _abi
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn((m, 512), generator=g).to(dtype).to(gpu)
+    w = torch.randint(-128, 128, (320, 512), generator=g, dtype=torch.int8).to(gpu)
+    b = None if bias is None else torch.randn(320, generator=g).to(bias).to(gpu)
+    wide = torch.zeros((m, 640), dtype=dtype, device=gpu)[:, :512]
+    wide.copy_(x)
+    for scale in ((torch.rand((320, 1), generator=g) * 1e-3).to(gpu), torch.tensor([1e-3], device=gpu)):
+        for rounded, epilogue, call in (
+                (False, kernels.EPI_ROW, lambda t: parallel_int8.row_linear(t, w, scale, None, 1, bias=b)),
+                (True, kernels.EPI_COLUMN,
+                 lambda t: dit_column_linear.column_linear(t, w, scale, out_dtype=dtype, bias=b))):
+            q, a = kernels.quantize_rows(x, convrot=True, round_rotated=rounded)
+            want = kernels.gemm(q, w, epilogue=epilogue, row_scale=a, col_scale=scale, bias=b, out_dtype=dtype)
+            assert torch.equal(_abi.native().linear(x, w, scale, b, epilogue, int(rounded), dtype), want)
+            got = call(x.view(1, m, 512))
+            assert got.shape == (1, m, 320) and got.dtype == dtype and torch.equal(got[0], want)
+            assert torch.equal(call(wide), want)
+    if m > 1:
+        assert _abi.native().linear(wide, w, scale, b, _abi.EPI_ROW, 0, dtype) is None
+    # what the native call refuses reaches the Python route's checks
+    with pytest.raises(ValueError):
+        dit_column_linear.column_linear(x, w, torch.ones(7, device=gpu))
+
+
+def test_native_attention_equals_two_calls(gpu):
+    from w8a8 import int8_attention as ia
+    g = torch.Generator().manual_seed(3)
+    packed = torch.randn((1, 150, 3 * 2 * 128), generator=g).half().to(gpu)
+    q, k, v = (packed[..., i * 256:(i + 1) * 256].view(1, 150, 2, 128).transpose(1, 2) for i in range(3))
+    for scale in (None, 0.05):
+        out = ia.int8_attention(q, k, v, scale=scale)
+        two = ia.int8_attention_from_prequantized(ia.prequantize_int8_attention(q, k, v, scale=scale))
+        assert out.is_contiguous() and torch.equal(out, two)
