@@ -203,10 +203,11 @@ __device__ __forceinline__ int readout_col(int nw, int h, int lane) {
   return nw + 64 * h + (lane % R::LPR) * R::CPL;
 }
 
-// Staged epilogue of one 128 x 32 NB quadrant (NB = 4, 3 or 2) through an
-// 8 KB wave-private LDS slice, in passes of 32 rows x 64 columns (8, or 4
-// for NB = 2). Each pass writes the raw int32 accumulators into the slice
-// (16-byte chunks XOR-swizzled by row), then
+// Staged epilogue of one 128 x 16 NR quadrant (NR = 8, 6, 4 or 3) through a
+// wave-private LDS slice (8 KB; 6 KB for NR = 3), in passes of 32 rows x up to
+// 64 columns (8, or 4 for NR <= 4). Each pass writes the raw int32
+// accumulators into the slice (16-byte chunks XOR-swizzled by row, or for the
+// 12 chunks of an NR = 3 row rotated by it), then
 // each lane reads CPL consecutive columns of one row back, dequantizes them
 // in the reference's order (ROW (C*a)*w, COLUMN C*(a*w), then + bias, then
 // the cast), adds the FP16 residual read with the same coalesced pattern
@@ -218,13 +219,14 @@ __device__ __forceinline__ int readout_col(int nw, int h, int lane) {
 // so the passes need only compiler ordering between the slice writes and
 // reads, and the next pass's writes may issue before this pass's reads
 // return.
-template <int EPI, int OUT, int FLAGS, bool INTERIOR, int NB = 4>
-__device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i (&acc)[2 * NB][8],
+template <int EPI, int OUT, int FLAGS, bool INTERIOR, int NR = 8>
+__device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i (&acc)[NR][8],
                                                         const float (&wsc)[2][8], const float (&bsc)[2][8],
                                                         const float (&as)[4], const int (&lbl)[4], int mw, int nw,
                                                         int lane, int8_t* stage, int64_t out_off) {
   using R = Readout<OUT>;
-  constexpr int RB = 256;  // 64 int32 per staged row
+  constexpr int RB = NR == 3 ? 192 : 256;  // 48 or 64 int32 per staged row
+  auto slot = [](int chunk, int row) { return (NR == 3 ? (chunk + row) % 12 : chunk ^ (row & 15)) << 4; };
   constexpr bool has_bias = (FLAGS & kWithBias) != 0;
   constexpr bool has_res = (FLAGS & kWithResidual) != 0;
   constexpr bool has_gate = (FLAGS & kWithGate) != 0;
@@ -238,7 +240,7 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i
     const int mb = pass >> 1, h = pass & 1;
     const int mrow = mw + mb * 32;
     const int ncol = nw + 64 * h + ocol;
-    const bool in_quad = NB != 3 || h == 0 || ocol < 32;
+    const bool in_quad = ocol < 16 * NR - 64 * h;
     const bool full_cols = INTERIOR || (p.vec16 && ncol + R::CPL <= p.n);
 #pragma unroll
     for (int it = 0; it < R::ITERS; ++it) {
@@ -265,21 +267,22 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i
 #pragma unroll
   for (int pass = 0; pass < 8; ++pass) {
     const int mb = pass >> 1, h = pass & 1;
-    // A quadrant 64 columns wide (NB == 2) has no second half.
-    if (NB == 2 && h == 1) continue;
+    // A quadrant at most 64 columns wide has no second half.
+    if (NR <= 4 && h == 1) continue;
     const int mrow = mw + mb * 32;
     const int ncol = nw + 64 * h + ocol;
-    // A quadrant 96 columns wide (NB == 3) has only its first 32 in the
-    // second half: the other read-out lanes of those passes store nothing.
-    const bool in_quad = NB != 3 || h == 0 || ocol < 32;
+    // A quadrant 96 columns wide (NR == 6) has only its first 32 in the
+    // second half, one of 48 (NR == 3) only those in the first: the other
+    // read-out lanes of these passes store nothing.
+    const bool in_quad = ocol < 16 * NR - 64 * h;
     // INTERIOR: every row and column of the quadrant is inside the output
     // and rows are 16-byte aligned, so no store needs a mask.
     const bool full_cols = INTERIOR || (p.vec16 && ncol + R::CPL <= p.n);
     // Buffer of pass q: the parity of its index among the passes that run
-    // (NB == 2 runs every other pass).
-    auto buf_of = [](int q) { return NB == 2 ? (q >> 1) & 1 : q & 1; };
+    // (NR <= 4 runs every other pass).
+    auto buf_of = [](int q) { return NR <= 4 ? (q >> 1) & 1 : q & 1; };
     if constexpr (kResAhead) {
-      const int next = NB == 2 ? pass + 2 : pass + 1;
+      const int next = NR <= 4 ? pass + 2 : pass + 1;
       if (next < 8) load_res(next, rbuf[buf_of(next)]);
     } else if constexpr (has_res) {
       load_res(pass, rbuf[0]);
@@ -321,9 +324,9 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i
     for (int ml = 0; ml < 2; ++ml)
 #pragma unroll
       for (int nl = 0; nl < 4; ++nl)
-        if (4 * h + nl < 2 * NB)
-          *reinterpret_cast<v4i*>(stage + (16 * ml + fr) * RB + (((4 * nl + fh) ^ fr) << 4)) =
-              acc[min(4 * h + nl, 2 * NB - 1)][2 * mb + ml];
+        if (4 * h + nl < NR)
+          *reinterpret_cast<v4i*>(stage + (16 * ml + fr) * RB + slot(4 * nl + fh, 16 * ml + fr)) =
+              acc[min(4 * h + nl, NR - 1)][2 * mb + ml];
     asm volatile("" ::: "memory");
     // Row scales of the lane's read-out rows (from the lanes holding them in
     // the MFMA layout), issued with the slice reads so one wait covers both.
@@ -336,8 +339,9 @@ __device__ __forceinline__ void store_quadrant32_passes(const GemmParams& p, v4i
       const int row = it * R::RPI + orow;
 #pragma unroll
       for (int q = 0; q < R::CPL / 4; ++q) {
-        const int chunk = ocol / 4 + q;
-        const v4i v = *reinterpret_cast<const v4i*>(stage + row * RB + ((chunk ^ (row & 15)) << 4));
+        // (lanes past an NR = 3 row read its last chunk and store nothing)
+        const int chunk = NR == 3 ? min(ocol / 4 + q, 11) : ocol / 4 + q;
+        const v4i v = *reinterpret_cast<const v4i*>(stage + row * RB + slot(chunk, row));
         c[it][4 * q] = v[0]; c[it][4 * q + 1] = v[1]; c[it][4 * q + 2] = v[2]; c[it][4 * q + 3] = v[3];
       }
     }
@@ -737,7 +741,7 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
   }
 }
 
-// Persistent GEMM (256 x 256, 256 x 192 or 128 x 256 output tiles) fed by
+// Persistent GEMM (256 x 256, 256 x 192, 128 x 256 or 128 x 192 output tiles) fed by
 // gfx950 direct global->LDS loads (global_load_lds_dwordx4). One workgroup
 // per CU walks its tiles; the operand stream runs across tile boundaries.
 //
@@ -757,7 +761,14 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
 // 128 x 256 tiles (a 48 KB stage, whose A tile would fill half a slot) take
 // a ring of three whole stages instead: stage g computes from slot g mod 3
 // while stage g + 1 lands and stage g + 2 streams into the slot stage g - 1
-// released, so two stages are in flight.
+// released, so two stages are in flight. 128 x 192 tiles (40 KB) take one of
+// four, three in flight: at a few hundred rows it puts more CUs to
+// work on a weight matrix (353 x 12800 x 5120: 201 instead of 150, 44.4 ->
+// 41.4 us) and may ask for a stage 2.5 stages ahead instead of 1.5. There the
+// CU's own rate of fetching lines binds (0.9 us a stage from HBM, 0.6 from
+// the last-level cache, with 67 workgroups as with 201): a fifth wavefront
+// that prefetched the weights into L2, and K walks that start at another
+// stage per column or row tile, were 0..30% slower.
 //
 // What bounds it: at the large shapes the board's power. The products run on
 // 16x16x64 MFMAs, which sustain 4260 TOPS (2.08 GHz) from one wave per SIMD
@@ -779,7 +790,8 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
 // stage returned), and before the epilogue vmcnt(NA + JB) (the tile's scale
 // and bias loads, issued before its K loop, have landed; only the two units
 // its last stage issued are younger): 8 / 16 for 256 x 256 and 8 / 14 for
-// 256 x 192 tiles. The three-stage ring waits vmcnt(NA + JB) = 12 at both.
+// 256 x 192 tiles. The three-stage ring waits vmcnt(NA + JB) = 12 at both, the
+// four-stage ring 2 (NA + JB) = 20 and NA + JB = 10.
 // Loads return in order, so a count is exact whenever at least that many
 // younger loads exist.
 //
@@ -859,31 +871,35 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <int EPI, int OUT, int FLAGS, int NB>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void gemm_i8_persistent(GemmParams p) {
-  // NR = 2 NB MFMA column blocks per wave. NB = 4 or 3: tiles are 256 x 64 NB
-  // (256 or 192 columns), the waves 2 x 2 quadrants of 128 x 32 NB. NB = 2:
-  // tiles are 128 x 256 (for M of a few hundred rows), the waves 1 x 4
-  // quadrants of 128 x 64 sharing the A tile, which fills half its slot. An
+  // NR MFMA column blocks of 16 per wave. NB = 4 or 3: tiles are 256 x 64 NB
+  // (256 or 192 columns), the waves 2 x 2 quadrants of 128 x 32 NB. NB = 2 or
+  // 1: tiles are 128 x 256 or 128 x 192 (for M of a few hundred rows), the
+  // waves 1 x 4 quadrants of 128 x 64 or 128 x 48 sharing the A tile. An
   // A unit is NA, a B unit JB DMA instructions per wave (8 rows each).
-  static_assert(NB == 4 || ((NB == 3 || NB == 2) && (FLAGS & kWithRope) == 0),
-                "NB 4, or 3 or 2 without the RoPE epilogue");
-  constexpr int BM = NB == 2 ? 128 : 256, BN = NB == 2 ? 256 : 64 * NB, WN = 32 * NB;
-  constexpr int NA = BM / 32, JB = BN / 32, NR = 2 * NB;
+  static_assert(NB == 4 || (NB >= 1 && NB <= 3 && (FLAGS & kWithRope) == 0),
+                "NB 4, or 3 to 1 without the RoPE epilogue");
+  constexpr int BM = plan_bm(NB), BN = plan_bn(NB), WN = BM == 128 ? BN / 4 : BN / 2;
+  constexpr int NA = BM / 32, JB = BN / 32, NR = WN / 16;
   extern __shared__ __attribute__((aligned(16))) int8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_m = (p.m + BM - 1) / BM, tiles_n = (p.n + BN - 1) / BN;
-  // Tile schedule. Workgroup w runs on XCD w % 8 (round-robin dispatch).
-  // With a grid that is a multiple of 8, XCD x owns the contiguous raster
-  // range [x*T/8, (x+1)*T/8) and its G/8 workgroups walk it in lockstep, so
-  // the tiles resident on one XCD at any time are raster neighbours sharing
-  // operand rows in that XCD's L2.
+  // Tile schedule. Workgroup w runs on XCD w % 8 (round-robin dispatch). XCD
+  // x owns a contiguous raster range of the items, in proportion to its
+  // workgroups (G / 8, one more for the first G % 8), which walk it in
+  // lockstep: the tiles resident on one XCD at any time are raster neighbours
+  // sharing operand rows in that XCD's L2. Grids that are no multiple of 8
+  // used to take the items in workgroup order, and the three row tiles of a
+  // 353-row product then fetched each weight tile into three L2s (353 x 12800
+  // x 5120 on 150 workgroups 46.2 -> 44.0 us).
   const int ksplit = max(p.ksplit, 1);
   const int total = tiles_m * tiles_n * ksplit, G = gridDim.x, w = blockIdx.x;
-  const bool by_xcd = (G & 7) == 0;
-  const int t_start = by_xcd ? (int)(((int64_t)(w & 7) * total) >> 3) : 0;
-  const int t_count = by_xcd ? (int)(((int64_t)((w & 7) + 1) * total) >> 3) - t_start : total;
-  const int t_stride = by_xcd ? G >> 3 : G;
-  const int t_first = by_xcd ? w >> 3 : w;
+  const int xcd = w & 7, gx = G >> 3, extra = G & 7;
+  const int before = xcd * gx + min(xcd, extra);   // workgroups of the XCDs before
+  const int t_stride = gx + (xcd < extra ? 1 : 0);
+  const int t_start = (int)((int64_t)total * before / G);
+  const int t_count = (int)((int64_t)total * (before + t_stride) / G) - t_start;
+  const int t_first = w >> 3;
   const int ntiles = t_first < t_count ? (t_count - t_first + t_stride - 1) / t_stride : 0;
   if (ntiles == 0) return;
   // Work item i of this workgroup: output tile item / ksplit, K split
@@ -955,7 +971,7 @@ void gemm_i8_persistent(GemmParams p) {
   // stage), lane (r = lane % 16, h = lane / 16) supplies row r, logical
   // chunk 4 u + h of both operands. Each wave holds an NR x 8 grid of 16x16
   // accumulator tiles (its 128 x 32 NB quadrant).
-  const int wm = NB == 2 ? 0 : wave >> 1, wn = NB == 2 ? wave : wave & 1;
+  const int wm = BM == 128 ? 0 : wave >> 1, wn = BM == 128 ? wave : wave & 1;
   const int fr = lane & 15, fh = lane >> 4;
   const int a_row = wm * 128 * kSK + fr * kSK, b_row = wn * WN * kSK + fr * kSK;
   // Fragment read I of sub-step u, in the order its first MFMA row consumes
@@ -1011,18 +1027,19 @@ void gemm_i8_persistent(GemmParams p) {
   // releases slots c, c + 1 (that row has consumed the stage's last
   // fragments), and unit 2g + 5 then goes to slot c.
   //
-  // 128 x 256 tiles (NB = 2) take a ring of three whole stages instead
-  // (STAGE_RING): stage slot s holds the A tile (16 KB) at 48 KB s and the
-  // B tile (32 KB) after it. Stage g computes from slot g mod 3; its first
-  // sub-step issues the B tile of stage g + 2 into the slot stage g - 1
-  // released (the A tile went there after that release), and after its own
-  // barrier it issues the A tile of stage g + 3 into its own slot: two stages
-  // (96 KB) in flight, where the five half-stage slots keep about one (their
-  // A slots half empty).
-  constexpr bool STAGE_RING = NB == 2;
+  // 128-row tiles take a ring of kRing whole stages instead: stage slot s
+  // holds the A tile (16 KB) at kStage2 s and the B tile after it. Stage g
+  // computes from slot g mod kRing; its first sub-step issues the B tile of
+  // stage g + kRing - 1 into the slot stage g - 1 released (the A tile went
+  // there after that release), and after its own barrier it issues the A tile
+  // of stage g + kRing into its own slot: kRing - 1 stages in flight (96 KB of
+  // 128 x 256 tiles, 120 KB of 128 x 192), where the five half-stage slots
+  // keep about one (their A slots half empty).
+  constexpr bool STAGE_RING = BM == 128;
   constexpr int kStage2 = (BM + BN) * kSK, kA2 = BM * kSK;
-  static_assert(!STAGE_RING || 3 * kStage2 <= kPersistentLds, "three stages fit the LDS");
-  auto next_slot = [](int slot) { return slot == (STAGE_RING ? 2 : kSlots - 1) ? 0 : slot + 1; };
+  constexpr int kRing = kPersistentLds / kStage2;   // whole stages that fit (STAGE_RING)
+  static_assert(!STAGE_RING || kRing == 3 || kRing == 4, "three or four stages fit the LDS");
+  auto next_slot = [](int slot) { return slot == (STAGE_RING ? kRing : kSlots) - 1 ? 0 : slot + 1; };
   // Byte offsets of the A and B tiles of the stage in slot s (STAGE_RING),
   // or whose A tile is in slot s (its B tile in the next slot).
   auto a_of = [&](int s) { return STAGE_RING ? s * kStage2 : s * kSTile; };
@@ -1033,7 +1050,11 @@ void gemm_i8_persistent(GemmParams p) {
   issue_unit(B_{}, b_of(STAGE_RING ? 1 : 2));
   if constexpr (STAGE_RING) {
     issue_unit(A_{}, a_of(2));
-    wait_vmcnt<2 * NA + JB>();  // stage 0 landed
+    if constexpr (kRing == 4) {
+      issue_unit(B_{}, b_of(2));
+      issue_unit(A_{}, a_of(3));
+    }
+    wait_vmcnt<(kRing - 1) * NA + (kRing - 2) * JB>();  // stage 0 landed
   } else {
     wait_vmcnt<NA + JB>();
   }
@@ -1076,9 +1097,9 @@ void gemm_i8_persistent(GemmParams p) {
     int ks = 0;
     do {  // nks >= 1
       // Slot of the next stage (its A tile), and the tile the first sub-step
-      // fills: the B tile of stage g + 2 (STAGE_RING) or unit 2g + 4.
+      // fills: the B tile of stage g + kRing - 1 (STAGE_RING) or unit 2g + 4.
       const int nxt = STAGE_RING ? next_slot(cur_a) : next_slot(next_slot(cur_a));
-      const int fill = STAGE_RING ? next_slot(nxt) : next_slot(next_slot(nxt));
+      const int fill = STAGE_RING ? (cur_a == 0 ? kRing - 1 : cur_a - 1) : next_slot(next_slot(nxt));
       const int ca = a_of(cur_a), cb = b_of(cur_a);
       using First = std::conditional_t<STAGE_RING, B_, A_>;
       using Second = std::conditional_t<STAGE_RING, A_, B_>;
@@ -1088,10 +1109,10 @@ void gemm_i8_persistent(GemmParams p) {
       substep(fa0, fb0, T0{}, [] {}, ca, cb, 1, fa1, fb1, First{}, fill_first);
       substep(fa1, fb1, T8{}, [&] {
         // The first row consumed the stage's last fragments. The next stage
-        // landed - only unit 2g + 4 (STAGE_RING: the A and B tiles of stage
-        // g + 2), issued after it, may still be in flight;
+        // landed - only unit 2g + 4 (STAGE_RING: the A and B tiles of stages
+        // g + 2 .. g + kRing - 1), issued after it, may still be in flight;
         __builtin_amdgcn_sched_barrier(0);
-        wait_vm_lgkm<STAGE_RING ? NA + JB : NA>();
+        wait_vm_lgkm<STAGE_RING ? (kRing - 2) * (NA + JB) : NA>();
         block_barrier();   // ... for every wave: the stage's slots are released.
       }, a_of(nxt), b_of(nxt), 0, fa0, fb0, Second{}, ca);
       stg = cb;
@@ -1115,7 +1136,7 @@ void gemm_i8_persistent(GemmParams p) {
     // the K loop, which needs them for its fragments.
     int elane = lane;
     __asm__ volatile("" : "+v"(elane));
-    int8_t* const stage_w = smem + stg + wave * 8192;
+    int8_t* const stage_w = smem + stg + wave * (NB == 1 ? JB * 1024 : 8192);
     const int64_t out_off = (item % ksplit) * p.split_stride;
     // Interior quadrants take a copy without store masks (not for the gate
     // variants, whose registers a second copy would push into spills).
@@ -1134,15 +1155,16 @@ void gemm_i8_persistent(GemmParams p) {
         store_quadrant_rope<EPI, kF16, false>(p, acc, wsc, as, mw, nw, elane, stage_w);
       }
     } else if ((FLAGS & kWithGate) == 0 && p.vec16 && mw + 128 <= p.m && nw + WN <= p.n)
-      store_quadrant32_passes<EPI, OUT, FLAGS, (FLAGS & kWithGate) == 0, NB>(p, acc, wsc, bsc, as, lbl, mw, nw,
+      store_quadrant32_passes<EPI, OUT, FLAGS, (FLAGS & kWithGate) == 0, NR>(p, acc, wsc, bsc, as, lbl, mw, nw,
                                                                             elane, stage_w, out_off);
     else
-      store_quadrant32_passes<EPI, OUT, FLAGS, false, NB>(p, acc, wsc, bsc, as, lbl, mw, nw, elane, stage_w,
+      store_quadrant32_passes<EPI, OUT, FLAGS, false, NR>(p, acc, wsc, bsc, as, lbl, mw, nw, elane, stage_w,
                                                           out_off);
     // The staging tile's next unit (2g + 6; STAGE_RING: the B tile of stage
-    // g + 3) is issued during the next stage; a wave's DMA into a slot
-    // writes the same 8 KB it used for staging, so its own staging reads
-    // returning is all that unit waits for.
+    // g + kRing) is issued during the next stage; a wave's DMA into a slot
+    // writes the same bytes it used for staging (8 KB; the 6 KB of its six
+    // instructions for 128 x 192 tiles), so its own staging reads returning
+    // is all that unit waits for.
     wait_lgkm();
     // The next tile's first fragments, read again (the last stage read them
     // too, but they would hold registers through the epilogue).
@@ -1611,13 +1633,14 @@ int launch_persistent(const GemmParams& p, int64_t tiles, int dev, hipStream_t s
   return W8A8_OK;
 }
 
-// The persistent kernel with 256 x 64 nb tiles.
+// The persistent kernel with the plan's tiles.
 template <int EPI, int OUT, int FLAGS>
 int launch_persistent_nb(const GemmParams& p, const GemmPlan& plan, int dev, hipStream_t s) {
   const int64_t tiles = plan_tiles(p.m, p.n, plan);
   if constexpr ((FLAGS & kWithRope) == 0) {
     if (plan.nb == 3) return launch_persistent<EPI, OUT, FLAGS, 3>(p, tiles, dev, s);
     if (plan.nb == 2) return launch_persistent<EPI, OUT, FLAGS, 2>(p, tiles, dev, s);
+    if (plan.nb == 1) return launch_persistent<EPI, OUT, FLAGS, 1>(p, tiles, dev, s);
   }
   return launch_persistent<EPI, OUT, FLAGS, 4>(p, tiles, dev, s);
 }

@@ -67,14 +67,18 @@ void launch_dequant(const GemmParams& p, const int32_t* acc, int64_t ldacc, hipS
 int gemm_ksplit(int64_t m, int64_t n, int64_t k, int dev, int64_t* workspace_bytes);
 
 // Tile shape and K split of the persistent kernel: nb 4: 256 x 256, nb 3:
-// 256 x 192, nb 2: 128 x 256 output tiles; K split ksplit ways.
+// 256 x 192, nb 2: 128 x 256, nb 1: 128 x 192 output tiles; K split ksplit
+// ways.
+constexpr int plan_bm(int nb) { return nb <= 2 ? 128 : 256; }
+constexpr int plan_bn(int nb) { return nb == 1 || nb == 3 ? 192 : 256; }
+
 struct GemmPlan {
   int nb;
   int ksplit;
 };
 
 inline int64_t plan_tiles(int64_t m, int64_t n, const GemmPlan& plan) {
-  const int64_t bm = plan.nb == 2 ? 128 : 256, bn = plan.nb == 2 ? 256 : 64 * plan.nb;
+  const int64_t bm = plan_bm(plan.nb), bn = plan_bn(plan.nb);
   return ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
 }
 
@@ -84,18 +88,21 @@ inline int64_t plan_tiles(int64_t m, int64_t n, const GemmPlan& plan) {
 // clock): rounds of work items x (stages per item x the tile's relative
 // cost + the tile's epilogue and the launch's fill and drain), plus the
 // split partials' write-and-read traffic at about 6.5 TB/s. A 256 x 192
-// stage costs 0.85 (0.80 of the cycles), a 128 x 256 stage 0.6 with an
-// epilogue of 6 instead of 8: fitted to the fastest measured plan of eight
-// shapes with M of 300..700 rows, where 256-row tiles leave most CUs idle
-// or need large split partials. A plan replaces the one before it only
+// stage costs 0.85 (0.80 of the cycles), a 128 x 256 stage 0.6 and a 128 x
+// 192 stage 0.48 with an epilogue of 6 instead of 8: fitted to the fastest
+// measured plan of shapes with M of 100..2048 rows, where 256-row tiles leave
+// most CUs idle or need large split partials. 128 x 192 against 128 x 256,
+// weights from HBM: 353 x 12800 x 5120 41.4 / 44.4 us, 256 x 14336 x 4096 30.3
+// / 32.6, 700 x 3072 x 3072 19.3 / 21.1, 1024 x 5120 x 5120 32.3 / 32.7; where
+// it would take a second round (512 x 14336 x 4096) 55.0 / 33.9. A plan replaces the one before it only
 // when it is 10% faster (256 x 256 and unsplit first).
 inline GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, int cus, int max_split = 8) {
   const int64_t kst = k / 128;
   GemmPlan best{4, 1};
   double best_t = -1.0;
-  for (int nb = 4; nb >= 2; --nb) {
+  for (int nb = 4; nb >= 1; --nb) {
     const int64_t tiles = plan_tiles(m, n, GemmPlan{nb, 1});
-    const double f = nb == 4 ? 1.0 : nb == 3 ? 0.85 : 0.6, e = nb == 2 ? 6.0 : 8.0;
+    const double f = nb == 4 ? 1.0 : nb == 3 ? 0.85 : nb == 2 ? 0.6 : 0.48, e = nb <= 2 ? 6.0 : 8.0;
     for (int ks = 1; ks <= max_split; ks *= 2) {
       if (ks > 1 && (tiles >= cus || kst / ks < 2)) break;
       const int64_t rounds = (tiles * ks + cus - 1) / cus;

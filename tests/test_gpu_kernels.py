@@ -308,6 +308,15 @@ def test_gemm_tile_shapes(gpu, m, n, k):
                           f'column {out_dtype}')
 
 
+@pytest.mark.parametrize('m,n,k', [(1000, 3000, 1536), (200, 1000, 512), (900, 5001, 1664), (100, 70000, 1536)])
+def test_gemm_128x192_tiles(gpu, m, n, k):
+    # Shapes the host plans with 128 x 192 tiles, on 256 CUs: ragged in both
+    # directions (last tiles of 104 rows and 120 columns), K split two ways,
+    # output rows that are not 16-byte aligned, and more tiles than CUs (365:
+    # the four-stage ring crosses tile boundaries). Every epilogue variant.
+    test_gemm_tile_shapes(gpu, m, n, k)
+
+
 def test_gemm_scalar_weight_scale_and_residual(gpu):
     g = torch.Generator().manual_seed(12)
     m, n, k = 130, 96, 512
