@@ -257,8 +257,6 @@ __device__ __forceinline__ int rha_code(float q) {
 // to a tie its nearest integer is the code; otherwise (12% of the waves on
 // random data), or when a scale is so large that its reciprocal is not a
 // normal number (wide), the wave divides. NaN gives -128 either way.
-constexpr float kWideScale = 0x1p120f;
-
 template <typename S, typename R>
 __device__ __forceinline__ void rha_codes32(const float (&x)[32], S&& s, R&& rcp, bool wide, uint32_t (&w)[8]) {
   float gap = 0.0f;

@@ -1,7 +1,8 @@
 // DiT modulated RMSNorm, optionally fused with ConvRot256 and the per-row
 // INT8 quantizer: the QKV / FC1 input preparation in one pass over x.
 //
-// One wavefront per row, lane l owning the 16-element units u = l + 64 j
+// One wavefront per row (a workgroup per row while the rows are few), lane l
+// of a wavefront owning the 16-element units u = l + 64 j
 // (elements [16u, 16u + 16)) as in the row quantizer, so loads and the int8
 // store are 128-bit and contiguous across the wave. The sum of squares has a
 // fixed order that does not depend on the launch: each lane adds its squares
@@ -11,6 +12,8 @@
 // square root followed by a correctly rounded division.
 #include "w8a8_device.h"
 #include "w8a8_host.h"
+
+#include <type_traits>
 
 namespace w8a8 {
 
@@ -56,8 +59,8 @@ __device__ __forceinline__ void load16_f32(const float* p, float (&v)[16]) {
 enum NormTables { kGain = 1, kMod = 2, kAnyTables = 4 };
 
 // v: x on entry; on return the normalized, modulated value rounded to DT
-// (as fp32), with its storage bits packed in bits.
-template <int DT, int TB>
+// (as fp32; times 1/16 when SCALED), with its storage bits packed in bits.
+template <int DT, int TB, bool SCALED>
 __device__ __forceinline__ void modulate16(float (&v)[16], uint32_t (&bits)[8], float inv, const float* w,
                                            const float* sh, const float* sc, int64_t c0) {
   const bool gain = (TB & kGain) || ((TB & kAnyTables) && w);
@@ -70,24 +73,29 @@ __device__ __forceinline__ void modulate16(float (&v)[16], uint32_t (&bits)[8], 
   }
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    float t = v[i] * inv;
+    float t = DT == kF16 ? mul_mix(v[i], inv) : v[i] * inv;
     if (gain) t = t * wv[i];
     if (mod) {
       const float f = 1.0f + scv[i];
       t = t * f;
       t = t + shv[i];
     }
-    uint16_t h;
-    if constexpr (DT == kF16) {
-      h = f2h_of_f32(t);
-      v[i] = h2f(h);
-    } else {
-      h = f2bf(t);
-      v[i] = bf2f(h);
-    }
-    if (i & 1) bits[i >> 1] |= (uint32_t)h << 16;
-    else bits[i >> 1] = h;
+    v[i] = t;
   }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    if constexpr (DT == kF16) {
+      bits[i] = f2h2_of_f32(v[2 * i], v[2 * i + 1]);
+      v[2 * i] = h2f((uint16_t)(bits[i] & 0xffffu));
+      v[2 * i + 1] = h2f((uint16_t)(bits[i] >> 16));
+    } else {
+      const uint16_t lo = f2bf(v[2 * i]), hi = f2bf(v[2 * i + 1]);
+      bits[i] = (uint32_t)lo | ((uint32_t)hi << 16);
+      v[2 * i] = bf2f(lo);
+      v[2 * i + 1] = bf2f(hi);
+    }
+  }
+  if constexpr (SCALED) scale16(v);
 }
 
 // Waves per workgroup of the norm-only kernel with AdaLN tables: the
@@ -103,15 +111,35 @@ constexpr int kNormStageMaxCols = 4096;   // 48 KB of tables
 template <int MODE, int W, bool STAGE>
 constexpr int norm_lds_floats(int cols) { return (rot_of<MODE>() ? W * kRotWave : 0) + (STAGE ? 3 * cols : 0); }
 
-template <int DT, int MODE, int J, int TB, int W = kNormWaves, bool STAGE = false>
-__global__ __launch_bounds__(64 * W) void norm_quant_kernel(NormParams p) {
+// SPLIT: a workgroup of J waves takes one row. Every wave adds all the squares
+// (the order is a chain through a lane's units), then normalizes, rotates and
+// quantizes unit wave j alone; the maxima meet in LDS. For few rows, where a
+// row per wave is one long chain of latencies on a part of the SIMDs. fp16
+// with AdaLN tables, row per wave / row per workgroup: 353 x 5120 15.2 / 7.4
+// us, 353 x 3072 10.5 / 6.3, 1024 x 5376 18.4 / 17.4, 1024 x 3072 10.9 / 7.9;
+// 2048 x 5376 22.9 / 29.9 and 2048 x 3072 12.9 / 13.0, where the squares added
+// J times over outweigh it: hence 1024 rows.
+constexpr int64_t kSplitRows = 1024;
+
+template <int DT, int MODE, int J, int TB, int W = kNormWaves, bool STAGE = false, bool SPLIT = false>
+__global__ __launch_bounds__(64 * W, J > 0 && J <= 6 && rot_of<MODE>() == 2 && DT == kF16 ? 4 : 1)
+void norm_quant_kernel(NormParams p) {
   constexpr int ROT = rot_of<MODE>();
+  constexpr bool PS = ROT != 0 && kPrescaled<DT>;
+  // Rotated fp16 values wait for the row's scale as the fp16 they are rounded
+  // to, eight registers a unit instead of sixteen; the maximum is taken on the
+  // fp32 rotation and rounded once (rounding is monotonic and odd). With x
+  // held in its storage type too, six units take 128 registers instead of 178:
+  // four waves per SIMD instead of two (6814 x 5376 73 -> 55 us).
+  constexpr bool KEEP16 = J > 0 && ROT == 2 && DT == kF16;
+  static_assert(!SPLIT || (W == J && !STAGE && MODE != 0), "one unit per wave");
+  __shared__ float wmax[SPLIT ? W : 1];
   static_assert(!STAGE || (TB == (kGain | kMod) && ROT == 0), "staged tables: norm-only DiT form");
   extern __shared__ __attribute__((aligned(16))) float dsm[];
   float* const lds = dsm;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t row0 = (int64_t)blockIdx.x * W;
-  const int64_t row = row0 + wave;
+  const int64_t row0 = SPLIT ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * W;
+  const int64_t row = SPLIT ? row0 : row0 + wave;
   float* const tw = dsm + (ROT ? W * kRotWave : 0);
   float* const tsc = tw + p.cols;
   float* const tsh = tsc + p.cols;
@@ -150,8 +178,8 @@ __global__ __launch_bounds__(64 * W) void norm_quant_kernel(NormParams p) {
   // Normalize one unit (v holds x), store y, rotate for the quantizer.
   auto finish = [&](int u, float (&v)[16], float inv, bool store_y) {
     uint32_t bits[8];
-    if (STAGE && staged) modulate16<DT, TB>(v, bits, inv, tw, tsh, tsc, (int64_t)u * 16);
-    else modulate16<DT, TB>(v, bits, inv, p.weight, sh, sc, (int64_t)u * 16);
+    if (STAGE && staged) modulate16<DT, TB, PS>(v, bits, inv, tw, tsh, tsc, (int64_t)u * 16);
+    else modulate16<DT, TB, PS>(v, bits, inv, p.weight, sh, sc, (int64_t)u * 16);
     if (store_y && yrow) {
       uint4* dst = reinterpret_cast<uint4*>(yrow + (int64_t)u * 16);
       dst[0] = make_uint4(bits[0], bits[1], bits[2], bits[3]);
@@ -159,8 +187,8 @@ __global__ __launch_bounds__(64 * W) void norm_quant_kernel(NormParams p) {
     }
     if constexpr (ROT != 0) {
       constexpr bool SG = (MODE & kNormSigned) != 0;
-      convrot256_lanes<true, SG>(v, buf, t, SG ? p.signs + 256 * (u >> 4) : nullptr);
-      if constexpr (ROT == 2) {
+      convrot256_lanes<true, SG, PS>(v, buf, t, SG ? p.signs + 256 * (u >> 4) : nullptr);
+      if constexpr (ROT == 2 && !KEEP16) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = round_to<DT>(v[i]);
       }
@@ -186,39 +214,70 @@ __global__ __launch_bounds__(64 * W) void norm_quant_kernel(NormParams p) {
   };
 
   if constexpr (J > 0) {
-    float v[J][16];
+    // The row waits in its storage type between the two passes over it.
+    uint4 raw[J][4];
     float ss = 0.0f;
 #pragma unroll
+    for (int j = 0; j < J; ++j)
+      if (lane + 64 * j < units) raw16<DT>(xrow + (int64_t)(lane + 64 * j) * 16, raw[j]);
+#pragma unroll
     for (int j = 0; j < J; ++j) {
-      const int u = lane + 64 * j;
-      if (u < units) {
-        load16<DT>(xrow + (int64_t)u * 16, v[j]);
-        ss = add_squares(ss, v[j]);
+      if (lane + 64 * j < units) {
+        float v[16];
+        unpack16<DT>(raw[j], v);
+        ss = add_squares(ss, v);
       }
     }
     const float inv = inv_rms(ss);
     float amax = 0.0f;
+    float keep[MODE != 0 && !KEEP16 ? J : 1][16];
+    uint32_t h16[KEEP16 ? J : 1][8];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       const int u = lane + 64 * j;
-      if (u < units) {
-        finish(u, v[j], inv, true);
+      if ((!SPLIT || j == wave) && u < units) {
+        float (&v)[16] = keep[MODE != 0 && !KEEP16 ? j : 0];
+        unpack16<DT>(raw[j], v);
+        finish(u, v, inv, true);
         if constexpr (MODE != 0) {
 #pragma unroll
-          for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[j][i]));
+          for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        }
+        if constexpr (KEEP16) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) h16[j][i] = f2h2_of_f32(v[2 * i], v[2 * i + 1]);
         }
       }
     }
     if constexpr (MODE != 0) {
       amax = wave_max(amax);
+      if constexpr (SPLIT) {
+        if (lane == 0) wmax[wave] = amax;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < J; ++j) amax = fmaxf(amax, wmax[j]);
+      }
+      if constexpr (KEEP16) amax = round_to<DT>(amax);
       const float s = row_scale_of(amax);
       const float rcp = 1.0f / s;
 #pragma unroll
       for (int j = 0; j < J; ++j) {
         const int u = lane + 64 * j;
-        if (u < units) store_q(u, v[j], s, rcp);
+        if ((!SPLIT || j == wave) && u < units) {
+          if constexpr (KEEP16) {
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              v[2 * i] = h2f((uint16_t)(h16[j][i] & 0xffffu));
+              v[2 * i + 1] = h2f((uint16_t)(h16[j][i] >> 16));
+            }
+            store_q(u, v, s, rcp);
+          } else {
+            store_q(u, keep[j], s, rcp);
+          }
+        }
       }
-      if (lane == 0) p.qscale[row] = s;
+      if (lane == 0 && (!SPLIT || wave == 0)) p.qscale[row] = s;
     }
   } else {
     // Rows too wide for registers: sum of squares, then absmax, then the
@@ -270,6 +329,25 @@ static void launch_norm_j(const NormParams& p, hipStream_t stream) {
   const int jneed = (int)(((p.cols >> 4) + 63) / 64);
   const dim3 grid((unsigned)((p.rows + W - 1) / W)), block(64 * W);
   const size_t lds = 4 * (size_t)max(norm_lds_floats<MODE, W, STAGE>((int)p.cols), 1);
+  if constexpr (MODE != 0 && !STAGE) {
+    // A row per workgroup while the rows are few.
+    if (jneed >= 2 && jneed <= 6 && p.rows <= kSplitRows) {
+      const dim3 rows((unsigned)p.rows);
+      auto go = [&](auto j_tag) {
+        constexpr int JJ = decltype(j_tag)::value;
+        hipLaunchKernelGGL((norm_quant_kernel<DT, MODE, JJ, TB, JJ, false, true>), rows, dim3(64 * JJ),
+                           4 * (size_t)max(norm_lds_floats<MODE, JJ, false>(0), 1), stream, p);
+      };
+      switch (jneed) {
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        case 3: go(std::integral_constant<int, 3>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 5: go(std::integral_constant<int, 5>{}); break;
+        default: go(std::integral_constant<int, 6>{}); break;
+      }
+      return;
+    }
+  }
 #define W8A8_NLAUNCH(JJ) hipLaunchKernelGGL((norm_quant_kernel<DT, MODE, JJ, TB, W, STAGE>), grid, block, lds, stream, p)
   switch (jneed) {
     case 1: W8A8_NLAUNCH(1); break;

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(
   auto load_unit = [&](int u, float (&v)[16]) {
     load16<DT>(xrow + (int64_t)u * 16 * dt_bytes<DT>(), v);
     if constexpr (RM != 0) {
-      convrot256_lanes<true, SG>(v, buf, t, smask(u));
+      if constexpr (kPrescaled<DT>) scale16(v);
+      convrot256_lanes<true, SG, kPrescaled<DT>>(v, buf, t, smask(u));
       if constexpr (RM == 2) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) v[i] = round_to<DT>(v[i]);
@@ -87,7 +88,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(
       float (&vj)[16] = v[KEEP16 ? 0 : j];
       unpack16<DT>(raw[j], vj);
       if constexpr (RM != 0) {
-        convrot256_lanes<true, SG>(vj, buf, t, smask(min(lane + 64 * j, units - 1)));
+        if constexpr (kPrescaled<DT>) scale16(vj);
+        convrot256_lanes<true, SG, kPrescaled<DT>>(vj, buf, t, smask(min(lane + 64 * j, units - 1)));
         if constexpr (RM == 2 && !KEEP16) {
 #pragma unroll
           for (int i = 0; i < 16; ++i) vj[i] = round_to<DT>(vj[i]);
@@ -190,7 +192,8 @@ __global__ __launch_bounds__(64 * W) void quantize_row_wg_kernel(
     if (u < units) {
       load16<DT>(xrow + (int64_t)u * 16 * dt_bytes<DT>(), v[j]);
       if constexpr (RM != 0) {
-        convrot256_lanes<true, SG>(v[j], buf, t, SG ? signs + 256 * (u >> 4) : nullptr);
+        if constexpr (kPrescaled<DT>) scale16(v[j]);
+        convrot256_lanes<true, SG, kPrescaled<DT>>(v[j], buf, t, SG ? signs + 256 * (u >> 4) : nullptr);
         if constexpr (RM == 2) {
 #pragma unroll
           for (int i = 0; i < 16; ++i) v[j][i] = round_to<DT>(v[j][i]);

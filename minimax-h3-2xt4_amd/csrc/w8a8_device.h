@@ -281,7 +281,9 @@ __device__ __forceinline__ float* rot_slot(float* lds, int wave, int lane) {
 // element, XORed into the values first: the rotation diag(s) then H, with s
 // a +-1 vector (exact: only signs change). A compile-time choice, so kernels
 // without signs hold no registers for them.
-template <bool NATURAL, bool SIGNS = false>
+// SCALED: v already carries the 1/16 (scale16 below): every sum is then the
+// unscaled one times 2^-4, so the results are the same bits.
+template <bool NATURAL, bool SIGNS = false, bool SCALED = false>
 __device__ __forceinline__ void convrot256_lanes(float (&v)[16], float* buf, int t,
                                                  const uint32_t* smask = nullptr) {
   if constexpr (SIGNS) {
@@ -311,8 +313,10 @@ __device__ __forceinline__ void convrot256_lanes(float (&v)[16], float* buf, int
   for (int b = 0; b < 4; ++b) h4(w[4 * b + 0], w[4 * b + 1], w[4 * b + 2], w[4 * b + 3]);
 #pragma unroll
   for (int b = 0; b < 4; ++b) h4(w[b + 0], w[b + 4], w[b + 8], w[b + 12]);
+  if constexpr (!SCALED) {
 #pragma unroll
-  for (int j = 0; j < 16; ++j) w[j] = w[j] * kInv16;
+    for (int j = 0; j < 16; ++j) w[j] = w[j] * kInv16;
+  }
   if constexpr (NATURAL) {
     // Each lane writes back exactly the floats it read (the transposed read
     // is a bijection), so no other lane's read can be overtaken.
@@ -332,8 +336,6 @@ __device__ __forceinline__ void convrot256_lanes(float (&v)[16], float* buf, int
   }
 }
 
-// The 16 int8 codes of elements 16t..16t+15 (natural order), packed for one
-// 16-byte store.
 // rne(x / s) as an fp32 integer value, without the clamp (quant1's rounding).
 __device__ __forceinline__ float quant_round(float x, float s, float rcp) {
   const float y = x * rcp;
@@ -342,20 +344,73 @@ __device__ __forceinline__ float quant_round(float x, float s, float rcp) {
   return n;
 }
 
-// Sixteen quant1 codes packed little-endian. v_cvt_pk_u8_f32 converts
-// n + 128 (exact: n is an integer) with saturation to [0, 255] and packs the
-// byte, so the clamp to [-128, 127] and the packing take one instruction per
-// code and the XOR with 0x80 turns the biased bytes into two's complement.
-// NaN converts to 0 (code -128) and +-inf saturate (127 / -128), as quant1's
-// clamp gives them.
+// Whether a rotation of DT inputs takes its 1/16 with their widening: fp16
+// values (2^-24 and up) stay exact at 2^-4 of their size, and the multiply
+// is the widening itself (v_fma_mix_f32). Smaller types' values could leave
+// the normal range.
+template <int DT>
+constexpr bool kPrescaled = DT == kF16;
+
+// -0, opaque to the compiler (which turns an FMA with a known -0 into a
+// conversion and a multiply).
+__device__ __forceinline__ float neg_zero() {
+  float z;
+  __asm__("s_brev_b32 %0, 1" : "=s"(z));
+  return z;
+}
+
+// a * b rounded once, as an FMA whose -0 addend changes neither the rounding
+// nor the sign of a zero: with a widened fp16 operand it is one v_fma_mix_f32.
+__device__ __forceinline__ float mul_mix(float a, float b) { return __builtin_fmaf(a, b, neg_zero()); }
+
+__device__ __forceinline__ void scale16(float (&v)[16]) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = mul_mix(v[i], kInv16);
+}
+
+// The 16 int8 codes of elements 16t..16t+15 (natural order), packed
+// little-endian for one 16-byte store. v_cvt_pk_u8_f32 rounds to nearest even
+// with saturation to [0, 255] and packs the byte, so the clamp to [-128, 127]
+// and the packing take one instruction per code and the XOR with 0x80 turns
+// the biased bytes into two's complement. z = x * rcp + 128 (one rounding) is
+// within 2^-16 of x / s + 128 for |x / s| < 128 (half an ulp of rcp and of z),
+// so unless some z of the wave lies within kNearTie of a tie (4% of the waves)
+// or the scale's reciprocal is not a normal number, it rounds as the quotient
+// does; otherwise the codes are taken again element by element with the
+// division where it decides. Beyond 128 both saturate to the same code, NaN
+// converts to 0 (code -128) and +-inf saturate, as quant1's clamp gives them.
+// One test for 16 codes, where a branch for each cost as much as the code
+// itself (with scale16 above, 6814 x 3584 fp16 rows rotated and
+// quantized 22.6 -> 20.4 us).
+constexpr float kNearTie = 1.25f / 65536.0f;
+constexpr float kWideScale = 0x1p120f;
+
 __device__ __forceinline__ uint4 quant16(const float (&v)[16], float s, float rcp) {
   uint32_t w[4];
+  float near = 1.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     uint32_t b = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) b = __builtin_amdgcn_cvt_pk_u8_f32(quant_round(v[4 * i + k], s, rcp) + 128.0f, k, b);
+    for (int k = 0; k < 4; ++k) {
+      const float z = __builtin_fmaf(v[4 * i + k], rcp, 128.0f);
+      near = fminf(near, fabsf(__builtin_amdgcn_fractf(z) - 0.5f));
+      b = __builtin_amdgcn_cvt_pk_u8_f32(z, k, b);
+    }
     w[i] = b ^ 0x80808080u;
+  }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(near < kNearTie || !(s < kWideScale)) != 0, 0)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t b = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float x = v[4 * i + k];
+        const float n = s < kWideScale ? quant_round(x, s, rcp) : rintf(x / s);
+        b = __builtin_amdgcn_cvt_pk_u8_f32(n + 128.0f, k, b);
+      }
+      w[i] = b ^ 0x80808080u;
+    }
   }
   return make_uint4(w[0], w[1], w[2], w[3]);
 }

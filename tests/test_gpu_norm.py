@@ -139,3 +139,18 @@ def test_norm_codes_equal_quantize_of_normalized_rows(gpu):
     r = kernels.norm_quantize(x, w, shift, scale, labels, eps=EPS, want_normalized=True)
     q, s = kernels.quantize_rows(r['y'], convrot=True, round_rotated=True)
     assert torch.equal(q, r['q']) and torch.equal(s, r['scale'])
+
+
+@pytest.mark.parametrize('rows,cols,mode', [(1024, 1280, 'rot'), (1025, 1280, 'rot'), (2, 2048, 'rot32'),
+                                            (1025, 4096, 'plain'), (3, 1296, 'plain'), (2, 5632, 'rot'),
+                                            (1025, 5632, 'rot')])
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_norm_row_per_workgroup_and_per_wave(gpu, rows, cols, mode, dtype):
+    """Both sides of the row count up to which a workgroup takes one row, at
+    two to six units a lane with whole and ragged last units."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x = randn16(g, (rows, cols), 4.0, dtype)
+    x[0, 5] *= 50
+    w, shift, scale, labels = _tables(g, cols, rows)
+    _check(_run(x, w, shift, scale, labels, mode, gpu), _oracle(x, w, shift, scale, labels, mode, dtype),
+           f'{rows}x{cols} {mode} {dtype}')
