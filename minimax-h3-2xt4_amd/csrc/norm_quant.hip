@@ -118,8 +118,8 @@ constexpr int norm_lds_floats(int cols) { return (rot_of<MODE>() ? W * kRotWave 
 // with AdaLN tables, row per wave / row per workgroup: 353 x 5120 15.2 / 7.4
 // us, 353 x 3072 10.5 / 6.3, 1024 x 5376 18.4 / 17.4, 1024 x 3072 10.9 / 7.9;
 // 2048 x 5376 22.9 / 29.9 and 2048 x 3072 12.9 / 13.0, where the squares added
-// J times over outweigh it: hence 1024 rows.
-constexpr int64_t kSplitRows = 1024;
+// J times over outweigh it: hence 768 rows.
+constexpr int64_t kSplitRows = 768;
 
 template <int DT, int MODE, int J, int TB, int W = kNormWaves, bool STAGE = false, bool SPLIT = false>
 __global__ __launch_bounds__(64 * W, J > 0 && J <= 6 && rot_of<MODE>() == 2 && DT == kF16 ? 4 : 1)
@@ -195,7 +195,8 @@ void norm_quant_kernel(NormParams p) {
     }
   };
   auto store_q = [&](int u, const float (&v)[16], float s, float rcp) {
-    *reinterpret_cast<uint4*>(p.q + row * p.ldq + (int64_t)u * 16) = quant16(v, s, rcp);
+    *reinterpret_cast<uint4*>(p.q + row * p.ldq + (int64_t)u * 16) =
+        ROT == 1 ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
   };
   // ss + x*x with one rounding: the square of a 16-bit float is exact in
   // fp32 (at most 22 significant bits, no overflow or underflow), so the FMA
@@ -214,8 +215,12 @@ void norm_quant_kernel(NormParams p) {
   };
 
   if constexpr (J > 0) {
-    // The row waits in its storage type between the two passes over it.
+    // The row waits in its storage type between the two passes over it (bf16
+    // rows of up to four units a lane widened, in the registers of their
+    // results: 16384 x 3072 64.5 us, 73.2 widened twice).
+    constexpr bool HOLD32 = DT == kBF16 && J <= 4 && MODE != 0;
     uint4 raw[J][4];
+    float keep[MODE != 0 && !KEEP16 ? J : 1][16];
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < J; ++j)
@@ -223,21 +228,21 @@ void norm_quant_kernel(NormParams p) {
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       if (lane + 64 * j < units) {
-        float v[16];
+        float tmp[16];
+        float (&v)[16] = HOLD32 ? keep[HOLD32 ? j : 0] : tmp;
         unpack16<DT>(raw[j], v);
         ss = add_squares(ss, v);
       }
     }
     const float inv = inv_rms(ss);
     float amax = 0.0f;
-    float keep[MODE != 0 && !KEEP16 ? J : 1][16];
     uint32_t h16[KEEP16 ? J : 1][8];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       const int u = lane + 64 * j;
       if ((!SPLIT || j == wave) && u < units) {
         float (&v)[16] = keep[MODE != 0 && !KEEP16 ? j : 0];
-        unpack16<DT>(raw[j], v);
+        if constexpr (!HOLD32) unpack16<DT>(raw[j], v);
         finish(u, v, inv, true);
         if constexpr (MODE != 0) {
 #pragma unroll

@@ -56,7 +56,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(
     }
   };
   auto store_unit = [&](int u, const float (&v)[16], float s, float rcp) {
-    *reinterpret_cast<uint4*>(q + row * ldq + (int64_t)u * 16) = quant16(v, s, rcp);
+    *reinterpret_cast<uint4*>(q + row * ldq + (int64_t)u * 16) =
+        RM == 1 ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
   };
 
   if constexpr (J > 0) {
@@ -220,7 +221,12 @@ __global__ __launch_bounds__(64 * W) void quantize_row_wg_kernel(
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     const int u = tid + 64 * W * j;
-    if (u < units) *reinterpret_cast<uint4*>(q + row * ldq + (int64_t)u * 16) = quant16(v[j], s, rcp);
+    // One test for sixteen codes shortens a lone row's chain (64 x 14336 fp32
+    // rotation 6.3 -> 5.4 us, 16 waves), not that of several rows on a CU (353
+    // x 5120 5.4 -> 6.2).
+    if (u < units)
+      *reinterpret_cast<uint4*>(q + row * ldq + (int64_t)u * 16) =
+          RM == 1 && W == 16 ? quant16(v[j], s, rcp) : quant16_each(v[j], s, rcp);
   }
   if (tid == 0) scale[row] = s;
 }

@@ -141,9 +141,9 @@ def test_norm_codes_equal_quantize_of_normalized_rows(gpu):
     assert torch.equal(q, r['q']) and torch.equal(s, r['scale'])
 
 
-@pytest.mark.parametrize('rows,cols,mode', [(1024, 1280, 'rot'), (1025, 1280, 'rot'), (2, 2048, 'rot32'),
-                                            (1025, 4096, 'plain'), (3, 1296, 'plain'), (2, 5632, 'rot'),
-                                            (1025, 5632, 'rot')])
+@pytest.mark.parametrize('rows,cols,mode', [(768, 1280, 'rot'), (769, 1280, 'rot'), (2, 2048, 'rot32'),
+                                            (769, 4096, 'plain'), (3, 1296, 'plain'), (2, 5632, 'rot'),
+                                            (769, 5632, 'rot')])
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 def test_norm_row_per_workgroup_and_per_wave(gpu, rows, cols, mode, dtype):
     """Both sides of the row count up to which a workgroup takes one row, at
