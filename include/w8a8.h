@@ -164,7 +164,8 @@ int w8a8_swiglu_quantize(const W8A8SwigluArgs* args);
  *          the 64 partials then meet in an xor butterfly (offsets 32..1)
  *   inv  = 1 / sqrt(ss * fp32(1/cols) + eps)      (IEEE sqrt and division)
  *   y    = x_dtype(((((x * inv) * w) * (1 + mod_scale[l])) + mod_shift[l]))
- * y: optional [rows, cols] x_dtype output of the normalized rows (ldy).
+ * y: optional [rows, cols] x_dtype output of the normalized rows (ldy); may
+ *   be x itself (ldy == ldx: in place).
  * convrot, round_rotated, q, ldq, q_scale, convrot_signs: as
  *   w8a8_quantize_rows applied to y. q NULL runs the norm alone (y
  *   required).

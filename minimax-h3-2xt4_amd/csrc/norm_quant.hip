@@ -35,6 +35,7 @@ struct NormParams {
   int64_t ldq;
   float* qscale;
   const uint32_t* signs;   // ConvRot sign words (0 or 0x80000000 per column), or null
+  bool shared;             // an output lies in x's memory (y == x: in place)
 };
 
 // MODE: 0 norm only, 1 quantize, 2 ConvRot256 (fp32) + quantize,
@@ -335,8 +336,9 @@ static void launch_norm_j(const NormParams& p, hipStream_t stream) {
   const dim3 grid((unsigned)((p.rows + W - 1) / W)), block(64 * W);
   const size_t lds = 4 * (size_t)max(norm_lds_floats<MODE, W, STAGE>((int)p.cols), 1);
   if constexpr (MODE != 0 && !STAGE) {
-    // A row per workgroup while the rows are few.
-    if (jneed >= 2 && jneed <= 6 && p.rows <= kSplitRows) {
+    // A row per workgroup while the rows are few; not in place, where a wave
+    // would store its unit while another still reads the row.
+    if (jneed >= 2 && jneed <= 6 && p.rows <= kSplitRows && !p.shared) {
       const dim3 rows((unsigned)p.rows);
       auto go = [&](auto j_tag) {
         constexpr int JJ = decltype(j_tag)::value;
@@ -383,6 +385,12 @@ static int launch_norm(const NormParams& p, hipStream_t stream) {
                        4 * (size_t)max(norm_lds_floats<MODE, kNormWaves, false>(0), 1), stream, p);
   }
   return launch_status("w8a8_norm_quantize");
+}
+
+// Whether [a, a + an) and [b, b + bn) share a byte.
+static bool spans_overlap(const void* a, int64_t an, const void* b, int64_t bn) {
+  const uintptr_t pa = (uintptr_t)a, pb = (uintptr_t)b;
+  return pa < pb + (uintptr_t)bn && pb < pa + (uintptr_t)an;
 }
 
 }  // namespace w8a8
@@ -442,6 +450,10 @@ extern "C" int w8a8_norm_quantize(const W8A8NormArgs* a) {
   p.q = a->q;
   p.ldq = a->ldq;
   p.qscale = a->q_scale;
+  const int64_t xbytes = ((a->rows - 1) * a->ldx + a->cols) * 2;
+  p.shared = (a->y && spans_overlap(a->x, xbytes, a->y, ((a->rows - 1) * a->ldy + a->cols) * 2)) ||
+             (a->q && (spans_overlap(a->x, xbytes, a->q, (a->rows - 1) * a->ldq + a->cols) ||
+                       spans_overlap(a->x, xbytes, a->q_scale, a->rows * 4)));
   W8A8_REQUIRE(a->convrot_signs == nullptr || (a->q && a->convrot && aligned16(a->convrot_signs)),
                "w8a8_norm_quantize: convrot_signs needs q, convrot and a 16-byte aligned array");
   p.signs = a->convrot_signs;

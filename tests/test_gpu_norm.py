@@ -6,7 +6,7 @@ import torch
 
 import oracle as o
 from helpers import assert_bits_equal, np_of, randn16, tname
-from w8a8 import kernels
+from w8a8 import _abi, kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -154,3 +154,22 @@ def test_norm_row_per_workgroup_and_per_wave(gpu, rows, cols, mode, dtype):
     w, shift, scale, labels = _tables(g, cols, rows)
     _check(_run(x, w, shift, scale, labels, mode, gpu), _oracle(x, w, shift, scale, labels, mode, dtype),
            f'{rows}x{cols} {mode} {dtype}')
+
+
+@pytest.mark.parametrize('rows,cols', [(353, 5120), (5, 1280), (1030, 3072), (9, 12288)])
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_norm_in_place(gpu, rows, cols, dtype):
+    """The C entry with y == x gives the bits of separate outputs, also at row
+    counts where a workgroup would share one row."""
+    g = torch.Generator().manual_seed(rows * 3 + cols)
+    x = randn16(g, (rows, cols), 4.0, dtype).to(gpu)
+    w, shift, scale, labels = (t.to(gpu) for t in _tables(g, cols, rows))
+    want = kernels.norm_quantize(x, w, shift, scale, labels, eps=EPS, want_normalized=True)
+    q = torch.empty((rows, cols), dtype=torch.int8, device=gpu)
+    qs = torch.empty((rows, 1), dtype=torch.float32, device=gpu)
+    _abi.call('w8a8_norm_quantize', _abi.NormArgs(
+        x_dtype=_abi.DTYPE_CODE[dtype], x=x.data_ptr(), ldx=cols, rows=rows, cols=cols, weight=w.data_ptr(),
+        mod_shift=shift.data_ptr(), mod_scale=scale.data_ptr(), ld_mod=cols, mod_rows=shift.shape[0], eps=EPS,
+        labels=labels.data_ptr(), y=x.data_ptr(), ldy=cols, convrot=256, round_rotated=1, q=q.data_ptr(), ldq=cols,
+        q_scale=qs.data_ptr(), stream=_abi.stream_of(x)))
+    assert torch.equal(x, want['y']) and torch.equal(q, want['q']) and torch.equal(qs, want['scale'])
