@@ -115,15 +115,33 @@ constexpr int norm_lds_floats(int cols) { return (rot_of<MODE>() ? W * kRotWave 
 // SPLIT: a workgroup of J waves takes one row. Every wave adds all the squares
 // (the order is a chain through a lane's units), then normalizes, rotates and
 // quantizes unit wave j alone; the maxima meet in LDS. For few rows, where a
-// row per wave is one long chain of latencies on a part of the SIMDs. fp16
-// with AdaLN tables, row per wave / row per workgroup: 353 x 5120 15.2 / 7.4
-// us, 353 x 3072 10.5 / 6.3, 1024 x 5376 18.4 / 17.4, 1024 x 3072 10.9 / 7.9;
-// 2048 x 5376 22.9 / 29.9 and 2048 x 3072 12.9 / 13.0, where the squares added
-// J times over outweigh it: hence 768 rows.
-constexpr int64_t kSplitRows = 768;
+// row per wave is one long chain of latencies on a part of the SIMDs; with
+// more, the squares added J times over outweigh it. Row per wave / per
+// workgroup, fp16 with AdaLN tables unless said: 353 x 5120 13.5 / 7.1 us, 353
+// x 3072 8.9 / 5.9. Rows of up to four units a lane: 1536 x 3072 11.5 / 10.8,
+// 1536 x 4096 14.6 / 12.5, 1536 x 3072 gain only 9.9 / 9.1, 1536 x 4096 bf16
+// 18.5 / 16.2; 2048 x 3072 12.4 / 13.2, 2048 x 4096 bf16 19.7 / 20.9. Five and
+// six units (a CU holds three such workgroups): 768 x 5376 16.9 / 12.4, 768 x
+// 5120 bf16 18.4 / 18.5; 896 x 5376 16.4 / 17.9, 896 x 5120 bf16 18.1 / 23.6.
+// Without the rounded rotation the chain is shorter (1536 x 4096 gain only,
+// fp32 rotation: 10.8 / 11.5), and the smaller line serves.
+constexpr int64_t split_rows(int jneed, int rot) { return jneed <= 4 && rot == 2 ? 1536 : 768; }
 
-template <int DT, int MODE, int J, int TB, int W = kNormWaves, bool STAGE = false, bool SPLIT = false>
-__global__ __launch_bounds__(64 * W, J > 0 && J <= 6 && rot_of<MODE>() == 2 && DT == kF16 ? 4 : 1)
+// WIDE: a rotated and rounded fp16 row waits for its scale as fp32, in the
+// registers its x was widened into while the squares are added, not as fp16
+// (KEEP16 below). Fewer conversions in a wave's chain, but more registers, so
+// it is the faster one while its waves all fit the SIMDs at once (KEEP16 /
+// WIDE, us): 2048 x 5376 21.5 / 21.1 and gain only 19.0 / 18.3, 2048 x 6144
+// signed 26.2 / 24.4, 3072 x 5376 gain only 23.7 / 22.7, 3072 x 4096 21.0 /
+// 20.6; past that 2560 x 5376 26.9 / 32.5, 4096 x 5376 gain only 27.9 / 31.4,
+// 4096 x 4096 26.0 / 28.3. Rows of one or two units fit four waves to a SIMD
+// either way and always take it (2048 x 2048 9.5 / 9.2, 8192 x 2048 23.5 /
+// 23.2).
+constexpr int64_t wide_rows(int j, int tables) { return j <= 2 ? INT64_MAX : j > 4 && (tables & kMod) ? 2048 : 3072; }
+
+template <int DT, int MODE, int J, int TB, int W = kNormWaves, bool STAGE = false, bool SPLIT = false,
+          bool WIDE = false>
+__global__ __launch_bounds__(64 * W, J > 0 && J <= 6 && rot_of<MODE>() == 2 && DT == kF16 && !WIDE ? 4 : 1)
 void norm_quant_kernel(NormParams p) {
   constexpr int ROT = rot_of<MODE>();
   constexpr bool PS = ROT != 0 && kPrescaled<DT>;
@@ -131,8 +149,10 @@ void norm_quant_kernel(NormParams p) {
   // to, eight registers a unit instead of sixteen; the maximum is taken on the
   // fp32 rotation and rounded once (rounding is monotonic and odd). With x
   // held in its storage type too, six units take 128 registers instead of 178:
-  // four waves per SIMD instead of two (6814 x 5376 73 -> 55 us).
-  constexpr bool KEEP16 = J > 0 && ROT == 2 && DT == kF16;
+  // four waves per SIMD instead of two (6814 x 5376 63 -> 48 us; with the sign
+  // words four registers spill there, 6144 x 6144 66 -> 61 us all the same).
+  constexpr bool KEEP16 = J > 0 && ROT == 2 && DT == kF16 && !WIDE;
+  static_assert(!WIDE || (J > 0 && ROT == 2 && DT == kF16 && !SPLIT), "the other storage of KEEP16's rows");
   static_assert(!SPLIT || (W == J && !STAGE && MODE != 0), "one unit per wave");
   __shared__ float wmax[SPLIT ? W : 1];
   static_assert(!STAGE || (TB == (kGain | kMod) && ROT == 0), "staged tables: norm-only DiT form");
@@ -197,7 +217,7 @@ void norm_quant_kernel(NormParams p) {
   };
   auto store_q = [&](int u, const float (&v)[16], float s, float rcp) {
     *reinterpret_cast<uint4*>(p.q + row * p.ldq + (int64_t)u * 16) =
-        ROT == 1 ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
+        ROT == 1 && (SPLIT || J != 2) ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
   };
   // ss + x*x with one rounding: the square of a 16-bit float is exact in
   // fp32 (at most 22 significant bits, no overflow or underflow), so the FMA
@@ -218,17 +238,22 @@ void norm_quant_kernel(NormParams p) {
   if constexpr (J > 0) {
     // The row waits in its storage type between the two passes over it (bf16
     // rows of up to four units a lane widened, in the registers of their
-    // results: 16384 x 3072 64.5 us, 73.2 widened twice).
-    constexpr bool HOLD32 = DT == kBF16 && J <= 4 && MODE != 0;
+    // results: 16384 x 3072 64.5 us, 73.2 widened twice; six units unrotated
+    // too, with 166 registers instead of 174 that is three waves to a SIMD and
+    // not two: 16384 x 5376 112 / 128 us).
+    constexpr bool HOLD32 = WIDE || (DT == kBF16 && MODE != 0 && (J <= 4 || MODE == 1));
     uint4 raw[J][4];
     float keep[MODE != 0 && !KEEP16 ? J : 1][16];
     float ss = 0.0f;
 #pragma unroll
     for (int j = 0; j < J; ++j)
-      if (lane + 64 * j < units) raw16<DT>(xrow + (int64_t)(lane + 64 * j) * 16, raw[j]);
+      if (!WIDE && lane + 64 * j < units) raw16<DT>(xrow + (int64_t)(lane + 64 * j) * 16, raw[j]);
+    // (WIDE: loads beside the adds, so that the first units' squares need not
+    // wait for the last: 2048 x 5376 gain only 18.9 -> 18.3 us.)
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       if (lane + 64 * j < units) {
+        if constexpr (WIDE) raw16<DT>(xrow + (int64_t)(lane + 64 * j) * 16, raw[j]);
         float tmp[16];
         float (&v)[16] = HOLD32 ? keep[HOLD32 ? j : 0] : tmp;
         unpack16<DT>(raw[j], v);
@@ -338,7 +363,7 @@ static void launch_norm_j(const NormParams& p, hipStream_t stream) {
   if constexpr (MODE != 0 && !STAGE) {
     // A row per workgroup while the rows are few; not in place, where a wave
     // would store its unit while another still reads the row.
-    if (jneed >= 2 && jneed <= 6 && p.rows <= kSplitRows && !p.shared) {
+    if (jneed >= 2 && jneed <= 6 && p.rows <= split_rows(jneed, rot_of<MODE>()) && !p.shared) {
       const dim3 rows((unsigned)p.rows);
       auto go = [&](auto j_tag) {
         constexpr int JJ = decltype(j_tag)::value;
@@ -355,17 +380,26 @@ static void launch_norm_j(const NormParams& p, hipStream_t stream) {
       return;
     }
   }
-#define W8A8_NLAUNCH(JJ) hipLaunchKernelGGL((norm_quant_kernel<DT, MODE, JJ, TB, W, STAGE>), grid, block, lds, stream, p)
+  auto go = [&](auto j_tag) {
+    constexpr int JJ = decltype(j_tag)::value;
+    if constexpr (DT == kF16 && rot_of<MODE>() == 2 && JJ > 0 && JJ <= 6) {
+      if (p.rows <= wide_rows(JJ, TB)) {
+        hipLaunchKernelGGL((norm_quant_kernel<DT, MODE, JJ, TB, W, STAGE, false, true>), grid, block, lds, stream, p);
+        return;
+      }
+    }
+    if constexpr (!(DT == kF16 && rot_of<MODE>() == 2) || JJ == 0 || JJ > 2)
+      hipLaunchKernelGGL((norm_quant_kernel<DT, MODE, JJ, TB, W, STAGE>), grid, block, lds, stream, p);
+  };
   switch (jneed) {
-    case 1: W8A8_NLAUNCH(1); break;
-    case 2: W8A8_NLAUNCH(2); break;
-    case 3: W8A8_NLAUNCH(3); break;
-    case 4: W8A8_NLAUNCH(4); break;
-    case 5: case 6: W8A8_NLAUNCH(6); break;
-    case 7: case 8: W8A8_NLAUNCH(8); break;
-    default: W8A8_NLAUNCH(0); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    case 4: go(std::integral_constant<int, 4>{}); break;
+    case 5: case 6: go(std::integral_constant<int, 6>{}); break;
+    case 7: case 8: go(std::integral_constant<int, 8>{}); break;
+    default: go(std::integral_constant<int, 0>{}); break;
   }
-#undef W8A8_NLAUNCH
 }
 
 // Rows held in registers for the DiT (gain + AdaLN tables) and plain

@@ -143,11 +143,15 @@ def test_norm_codes_equal_quantize_of_normalized_rows(gpu):
 
 @pytest.mark.parametrize('rows,cols,mode', [(768, 1280, 'rot'), (769, 1280, 'rot'), (2, 2048, 'rot32'),
                                             (769, 4096, 'plain'), (3, 1296, 'plain'), (2, 5632, 'rot'),
-                                            (769, 5632, 'rot')])
+                                            (769, 5632, 'rot'), (1536, 3072, 'rot'), (1537, 3072, 'rot'),
+                                            (1537, 3840, 'rot'), (3072, 2304, 'rot'), (3073, 2304, 'rot'),
+                                            (2048, 5120, 'rot'), (2049, 5120, 'rot'), (2049, 1536, 'rot'),
+                                            (769, 1536, 'rot32')])
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 def test_norm_row_per_workgroup_and_per_wave(gpu, rows, cols, mode, dtype):
-    """Both sides of the row count up to which a workgroup takes one row, at
-    two to six units a lane with whole and ragged last units."""
+    """Both sides of the row counts up to which a workgroup takes one row and
+    up to which fp16 rows wait as fp32, at two to six units a lane with whole
+    and ragged last units."""
     g = torch.Generator().manual_seed(rows + cols)
     x = randn16(g, (rows, cols), 4.0, dtype)
     x[0, 5] *= 50
@@ -173,3 +177,22 @@ def test_norm_in_place(gpu, rows, cols, dtype):
         labels=labels.data_ptr(), y=x.data_ptr(), ldy=cols, convrot=256, round_rotated=1, q=q.data_ptr(), ldq=cols,
         q_scale=qs.data_ptr(), stream=_abi.stream_of(x)))
     assert torch.equal(x, want['y']) and torch.equal(q, want['q']) and torch.equal(qs, want['scale'])
+
+
+@pytest.mark.parametrize('rows,cols', [(2, 256), (1600, 1536), (1600, 2304), (3080, 4096), (1030, 5376), (2100, 5376)])
+@pytest.mark.parametrize('form', ['gain', 'signed'])
+def test_norm_storage_forms(gpu, rows, cols, form):
+    """fp16 rows held as fp32 and as fp16, without AdaLN tables and with the
+    sign words: the codes of quantizing the kernel's own normalized rows."""
+    g = torch.Generator().manual_seed(rows * 5 + cols)
+    x = randn16(g, (rows, cols), 4.0).to(gpu)
+    w, shift, scale, labels = (t.to(gpu) for t in _tables(g, cols, rows))
+    signs = None
+    if form == 'gain':
+        shift = scale = labels = None
+    else:
+        signs = (torch.randint(0, 2, (cols,), generator=g, dtype=torch.int32) << 31).to(gpu)
+    r = kernels.norm_quantize(x, w, shift, scale, labels, eps=EPS, want_normalized=True, signs=signs)
+    y = kernels.norm_quantize(x, w, shift, scale, labels, eps=EPS, quantize=False)['y']
+    q, s = kernels.quantize_rows(y, convrot=True, round_rotated=True, signs=signs)
+    assert torch.equal(r['y'], y) and torch.equal(r['q'], q) and torch.equal(r['scale'], s)
