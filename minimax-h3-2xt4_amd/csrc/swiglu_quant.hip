@@ -67,12 +67,14 @@ __global__ __launch_bounds__(64 * W) void swiglu_quant_kernel(
     return m;
   };
   auto store_group = [&](int g, const float (&v)[16], float s, float rcp) {
-    // One test for sixteen codes (quant16) shortens a lone row's chain (64 x
-    // 14336 9.3 -> 8.2 us) but slows a full GPU, tested one by one against it:
-    // 16384 x 4096 76.1 / 80.3 us, 6814 x 7168 63.0 / 64.9, 16384 x 2048 41.6 /
-    // 43.2.
+    // One test for sixteen codes (quant16) shortens a lone row's chain while a
+    // lane holds one group of it (64 x 14336 9.1 -> 8.2 us). With more groups
+    // a second copy of each weighs more (one by one / one test: 64 x 28672 11.9
+    // / 12.8 us, 256 x 28672 14.9 / 16.0, 64 x 57344 fp32 27.6 / 28.3), and so it
+    // does on a full GPU: 16384 x 4096 76.1 / 80.3, 6814 x 7168 63.0 / 64.9,
+    // 16384 x 2048 41.6 / 43.2.
     *reinterpret_cast<uint4*>(q + row * ldq + (int64_t)g * 256 + 16 * t) =
-        W == 16 ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
+        W == 16 && P == 1 ? quant16(v, s, rcp) : quant16_each(v, s, rcp);
   };
   auto row_reduce = [&](float m) {
     m = wave_max(m);
