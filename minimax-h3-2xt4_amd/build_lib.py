@@ -6,10 +6,13 @@ and csrc/native.cpp (host C++ on torch's tensors) into the module _native.
 Each csrc/*.hip compiles to an object under _build/ (in parallel), then one
 hipcc link produces w8a8/libw8a8.so next to the Python bindings.
 csrc/gemm_inst.hip compiles once per (epilogue, output dtype) pair of the
-GEMM (INST_VARIANTS), each with its own -D pair.
+GEMM (INST_VARIANTS), each with its own -D pair. The library needs neither
+torch nor Python's headers: it is linked whatever becomes of _native, which is
+left out where torch is not installed (only the Python package loads it).
 """
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
@@ -112,23 +115,23 @@ def _link_native(obj, verbose):
     os.replace(tmp, NATIVE_OUT)
 
 
+def _link(objs, verbose):
+    tmp = OUT.with_suffix('.so.tmp')
+    _run([hipcc(), f'--offload-arch={ARCH}', '-shared', '-fPIC', *map(str, objs), '-o', str(tmp)], 'link', verbose)
+    os.replace(tmp, OUT)
+
+
 def build(jobs=None, verbose=False):
     BUILD.mkdir(exist_ok=True)
     units = _units()
     jobs = jobs or min(len(units) + 1, max(1, os.cpu_count() or 4))
+    with_native = importlib.util.find_spec('torch') is not None
     with cf.ThreadPoolExecutor(max_workers=jobs) as pool:
-        native = pool.submit(_compile_native, verbose)
+        native = pool.submit(_compile_native, verbose) if with_native else None
         objs = list(pool.map(lambda u: _compile(u, verbose), units))
-        native = native.result()
-    tmp = OUT.with_suffix('.so.tmp')
-    cmd = [hipcc(), f'--offload-arch={ARCH}', '-shared', '-fPIC', *map(str, objs), '-o', str(tmp)]
-    if verbose:
-        print(' '.join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f'link failed:\n{res.stdout}\n{res.stderr}')
-    os.replace(tmp, OUT)
-    _link_native(native, verbose)
+    _link(objs, verbose)
+    if with_native:
+        _link_native(native.result(), verbose)
     return OUT
 
 
