@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define W8A8_ABI_VERSION 13
+#define W8A8_ABI_VERSION 14
 
 typedef enum w8a8_status {
   W8A8_OK = 0,
@@ -498,7 +498,7 @@ int w8a8_dequantize(const W8A8DequantArgs* args);
 int w8a8_segment_labels(const int32_t* ends, const int32_t* values, int64_t count, int32_t* labels, int64_t rows,
                         void* stream);
 
-/* ABI version (W8A8_ABI_VERSION). */
+/* ABI version (W8A8_ABI_VERSION; 14 added w8a8_segment_labels). */
 int w8a8_abi_version(void);
 
 /* sizeof of each argument struct, by index: 0 Quant, 1 Swiglu, 2 Gemm,

@@ -15,7 +15,7 @@ LIB_PATH = Path(__file__).resolve().parent / 'libw8a8.so'
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_LAUNCH = 0, 1, 2, 3
 F16, BF16, F32, I32, I8 = 1, 2, 3, 4, 5
 EPI_INT32, EPI_ROW, EPI_COLUMN = 0, 1, 2
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _c = ctypes
 _p = ctypes.c_void_p
@@ -120,7 +120,10 @@ def load(path=None):
         raise RuntimeError(f'{p} is missing: build it with python minimax-h3-2xt4_amd/build_lib.py '
                            '(there is no CPU fallback for the W8A8 path)')
     lib = ctypes.CDLL(os.fspath(p))
+    # The version first: a library of another one may lack the symbols below.
     lib.w8a8_abi_version.restype = _c.c_int
+    if lib.w8a8_abi_version() != ABI_VERSION:
+        raise RuntimeError(f'libw8a8 ABI {lib.w8a8_abi_version()} != {ABI_VERSION}')
     lib.w8a8_struct_size.restype = _c.c_int64
     lib.w8a8_struct_size.argtypes = [_c.c_int32]
     lib.w8a8_last_error.restype = _c.c_char_p
@@ -134,8 +137,6 @@ def load(path=None):
         fn = getattr(lib, name)
         fn.restype = _c.c_int
         fn.argtypes = [ctypes.POINTER(st)]
-    if lib.w8a8_abi_version() != ABI_VERSION:
-        raise RuntimeError(f'libw8a8 ABI {lib.w8a8_abi_version()} != {ABI_VERSION}')
     for i, st in enumerate(STRUCTS):
         if lib.w8a8_struct_size(i) != ctypes.sizeof(st):
             raise RuntimeError(f'{st.__name__}: library size {lib.w8a8_struct_size(i)} != '

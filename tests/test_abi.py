@@ -3,6 +3,7 @@ declares, agrees on struct layouts, and rejects invalid arguments before any
 launch (nothing here runs device code)."""
 import ctypes
 import re
+import subprocess
 from pathlib import Path
 
 import pytest
@@ -37,6 +38,15 @@ def test_version_and_struct_sizes():
     # header field order: sizes computed from the C declaration
     assert [ctypes.sizeof(s) for s in _abi.STRUCTS] == [104, 104, 192, 144, 152, 104, 224, 144]
     assert ctypes.sizeof(_abi.RopeEpilogue) == 48   # static_assert'ed in the library too
+
+
+def test_library_of_another_version_is_named(tmp_path):
+    # An older library has neither the newer symbols nor this version.
+    src, lib = tmp_path / 'old.c', tmp_path / 'libold.so'
+    src.write_text('int w8a8_abi_version(void) { return 13; }\n')
+    subprocess.run(['gcc', '-shared', '-fPIC', str(src), '-o', str(lib)], check=True)
+    with pytest.raises(RuntimeError, match='libw8a8 ABI 13 != '):
+        _abi.load(lib)
 
 
 def _expect_invalid(name, args, fragment):
