@@ -157,8 +157,10 @@ def labels_for(rows, segments, modulation_rows=9, device=None):
     """int32 [rows] gate-table row of every row, or None when the segments do
     not tile the rows (patches/tilelang_dit_fusion.py:106-124). On the current
     GPU a kernel writes them (no copy from the host, which would wait for the
-    stream)."""
-    if isinstance(device, torch.device) and device.type == 'cuda' and device.index is not None:
+    stream); before torch has initialised one, the copy does that, or says why
+    it cannot."""
+    if (isinstance(device, torch.device) and device.type == 'cuda' and device.index is not None
+            and torch.cuda.is_initialized()):
         labels = _abi.native().segment_labels(rows, segments, modulation_rows, device.index)
         if labels is not None:
             return labels

@@ -100,6 +100,12 @@ def test_segment_labels():
     assert labels_for(5, [(0, 4, 1)]) is None
 
 
+def test_segment_labels_need_no_gpu_to_refuse():
+    # Segments that do not tile the rows give None, whether or not a GPU is there.
+    from w8a8.h3_tensor_flow import labels_for
+    assert labels_for(5, [(0, 4, 1)], device=torch.device('cuda', 0)) is None
+
+
 def test_output_buffers_are_validated_before_any_launch():
     x = torch.randn(8, 256).half()
     with pytest.raises(ValueError, match='out must be int8'):
