@@ -50,6 +50,11 @@ INST_VARIANTS = [(0, 4), (1, 1), (1, 2), (1, 3), (2, 1), (2, 2), (2, 3)]
 FILE_FLAGS = {'attention.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form']}
 
 
+# Kernels whose MFMAs come from inline assembly: mfma_hazards.py checks the
+# assembly that the compiler made of them, and the build fails on a hazard.
+CHECKED_KERNELS = {'gemm_inst.hip': 'gemm_i8_persistent'}
+
+
 def hipcc():
     path = shutil.which('hipcc') or '/opt/rocm/bin/hipcc'
     if not Path(path).exists():
@@ -70,26 +75,35 @@ def _units():
     return units
 
 
-def _compile(unit, verbose):
-    src, name, extra = unit
-    obj = BUILD / name
-    cmd = [hipcc(), *HIPCC_FLAGS, *extra, '-c', str(src), '-o', str(obj)]
-    if verbose:
-        print(' '.join(cmd), flush=True)
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f'hipcc failed for {src.name}:\n{res.stdout}\n{res.stderr}')
-    if verbose and res.stderr.strip():
-        print(res.stderr, file=sys.stderr)
-    return obj
-
-
 def _run(cmd, what, verbose):
     if verbose:
         print(' '.join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f'{what} failed:\n{res.stdout}\n{res.stderr}')
+    if verbose and res.stderr.strip():
+        print(res.stderr, file=sys.stderr)
+
+
+def _compile(unit, verbose):
+    src, name, extra = unit
+    obj = BUILD / name
+    checked = CHECKED_KERNELS.get(src.name)
+    if checked is None:
+        _run([hipcc(), *HIPCC_FLAGS, *extra, '-c', str(src), '-o', str(obj)], f'hipcc {src.name}', verbose)
+        return obj
+    # The assembly is kept (the compiler's temporaries take the output's
+    # folder) until the check below has read it.
+    tmp = BUILD / f'{obj.stem}.tmp'
+    shutil.rmtree(tmp, ignore_errors=True)
+    tmp.mkdir()
+    _run([hipcc(), *HIPCC_FLAGS, *extra, '-save-temps=obj', '-c', str(src), '-o', str(tmp / name)],
+         f'hipcc {src.name}', verbose)
+    asm, = tmp.glob(f'*{ARCH}*.s')
+    _run([sys.executable, str(PKG / 'mfma_hazards.py'), str(asm), checked], f'wait states of {name}', verbose)
+    os.replace(tmp / name, obj)
+    shutil.rmtree(tmp)
+    return obj
 
 
 def _compile_native(verbose):

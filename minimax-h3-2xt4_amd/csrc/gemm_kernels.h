@@ -825,9 +825,12 @@ __device__ __forceinline__ int lds_chunk(int row, int c) { return c ^ ((row >> 1
 // builtin lets the compiler pick another destination, and with all 256
 // accumulator registers taken it then copies tuples around in the K loop
 // (some 300 v_accvgpr moves per stage). The compiler knows neither that this
-// is an MFMA nor its wait states: accumulators written by other instructions
-// settle before the first one (acc_zero), and none is read before
-// acc_ready; the fragments come from LDS reads, whose waits it does count.
+// is an MFMA nor its wait states. So a and b must come from LDS reads (whose
+// waits it does count): a VALU write to them, such as a copy or a reload,
+// needs two wait states before the MFMA. Accumulators written by other
+// instructions settle before the first one (acc_zero), and none is read
+// before acc_ready. The build checks the assembly for all three
+// (mfma_hazards.py).
 __device__ __forceinline__ void mfma_tied(v4i& acc, const v4i& a, const v4i& b) {
   __asm__("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
