@@ -24,6 +24,7 @@
 // probabilities are then already the B operand of O^T = V^T.P^T; the signed
 // MFMA takes P - 128, and its accumulator starts from the block's 128 * sum
 // of V codes, so it ends with the exact P.V.
+#include "attn_plan.h"
 #include "w8a8_device.h"
 #include "w8a8_host.h"
 
@@ -35,8 +36,6 @@ namespace w8a8 {
 constexpr int kAttnD = 128;        // head dimension
 constexpr int kAttnBK = 128;       // keys per block (the reference launcher's CTA_K = 128)
 constexpr int kAttnChunk = 256;    // tokens per partial of the key statistics
-constexpr int kAttnWaveQ = 32;     // queries per wavefront
-constexpr int kAttnWaves = 4;      // wavefronts per workgroup (one per SIMD; two workgroups per CU)
 constexpr int kAttnBQ = kAttnWaves * kAttnWaveQ;   // queries per workgroup
 constexpr int kAttnTile = kAttnBK * kAttnD;        // bytes of one K or V^T tile
 constexpr int kAttnDmaTile = kAttnTile / 1024 / kAttnWaves;   // 1 KB DMA instructions per wave and tile
@@ -1018,21 +1017,6 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attention_split_kernel(Att
       }
     }
   }
-}
-
-// Whether the split kernel is the faster one, from both kernels' measured times
-// in tenths of a microsecond: a round of split workgroups (one per CU) costs
-// 4.5 us and 2.6 us for each step of its longest wave, the other kernel 14 us
-// and 2.6 us a block while its grid fits the GPU. Both sides (us, plain and
-// split): 16 heads x 353 x 1000 27.9 / 12.5, 8 x 64 x 32768 540 / 188, 28 x 350
-// x 256 15.6 / 14.0, 28 x 700 x 256 19.5 / 20.1, 20 x 1000 x 512 26.1 / 22.2,
-// 28 x 1100 x 512 28.7 / 31.0, 24 x 700 x 3000 68.7 / 65.3, 12 x 2000 x 2000
-// 52.0 / 50.4, 16 x 2000 x 2000 55.0 / 65.5. A single block has nothing to
-// split (28 x 700 x 128 9.0 / 20.2).
-static bool split_wins(int64_t nq, int64_t bh, int64_t nblk, int64_t cus) {
-  if (nblk < 2) return false;
-  const int64_t rounds = ((nq + kAttnWaveQ - 1) / kAttnWaveQ * bh + cus - 1) / cus;
-  return rounds * (45 + 26 * ((nblk + kAttnWaves - 1) / kAttnWaves)) < 140 + 26 * nblk;
 }
 
 static int64_t attn_chunks(int64_t nk) { return (nk + kAttnChunk - 1) / kAttnChunk; }

@@ -95,16 +95,22 @@ inline int64_t plan_tiles(int64_t m, int64_t n, const GemmPlan& plan) {
 // weights from HBM: 353 x 12800 x 5120 41.4 / 44.4 us, 256 x 14336 x 4096 30.3
 // / 32.6, 700 x 3072 x 3072 19.3 / 21.1, 1024 x 5120 x 5120 32.3 / 32.7; where
 // it would take a second round (512 x 14336 x 4096) 55.0 / 33.9. A plan replaces the one before it only
-// when it is 10% faster (256 x 256 and unsplit first).
+// when it is 10% faster (256 x 256 and unsplit first). The cost knows neither
+// the finishing kernel's launch nor its reads, so 128 x 192 tiles split K only
+// where the plan they replace does, and eight ways only where it does that
+// (this way / by the cost alone, over 220 shapes whose plan the tile changes:
+// 510 x 512 x 640 10.2 / 14.3 us, 1376 x 512 x 1152 12.7 / 17.0, 160 x 512 x
+// 2304 12.3 / 14.6; two ways to four stays, 0.95 of the time on average).
 inline GemmPlan gemm_plan(int64_t m, int64_t n, int64_t k, int cus, int max_split = 8) {
   const int64_t kst = k / 128;
   GemmPlan best{4, 1};
   double best_t = -1.0;
   for (int nb = 4; nb >= 1; --nb) {
     const int64_t tiles = plan_tiles(m, n, GemmPlan{nb, 1});
+    const int cap = nb > 1 || best.ksplit == 8 ? 8 : best.ksplit == 1 ? 1 : 4;
     const double f = nb == 4 ? 1.0 : nb == 3 ? 0.85 : nb == 2 ? 0.6 : 0.48, e = nb <= 2 ? 6.0 : 8.0;
     for (int ks = 1; ks <= max_split; ks *= 2) {
-      if (ks > 1 && (tiles >= cus || kst / ks < 2)) break;
+      if (ks > 1 && (tiles >= cus || kst / ks < 2 || ks > cap)) break;
       const int64_t rounds = (tiles * ks + cus - 1) / cus;
       double t = (double)rounds * ((double)((kst + ks - 1) / ks) * f + e);
       if (ks > 1) t += (double)ks * m * n * 8 / 6.5e12 * 1e6;
