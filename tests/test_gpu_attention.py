@@ -20,11 +20,10 @@ SHAPES = [
     (2, 3, 200, 64, torch.float32),
     (1, 1, 128, 300, torch.float16),
     (1, 2, 257, 1000, torch.float16),
-    # the step loop's two-step unroll and every tail (13, 14 and 15 blocks:
-    # after the loop one or no further step, then the step whose next block
-    # is the last, alternating tiles), key counts that are and are not
-    # multiples of 128, and long sequences (queries are independent, so a
-    # short query set exercises the whole key loop)
+    # 13, 14 and 15 key blocks, key counts that are and are not multiples of
+    # 128, and long sequences (queries are independent, so a short query set
+    # exercises the whole key loop). One or two heads of few queries take the
+    # kernel that splits the keys over a workgroup's waves, from two blocks on.
     (1, 1, 64, 1600, torch.float16),
     (1, 1, 33, 1664, torch.float16),
     (1, 1, 40, 1792, torch.float16),
@@ -210,16 +209,28 @@ def test_prepare_ties_and_wide_scales(gpu):
         assert np_of(prep[name]).tobytes() == np.ascontiguousarray(want[name]).tobytes(), name
 
 
-@pytest.mark.parametrize('nq,nk', [(33, 1600), (64, 1664), (40, 1792), (33, 1920), (32, 130), (200, 64)])
-def test_both_kernels_match_oracle(gpu, nq, nk):
-    """260 heads fill the GPU with 128-query workgroups; one head alone takes
-    the kernel that splits the keys over a workgroup's waves. Both follow the
-    oracle, at every tail of the step loop (one to three waves without a last
-    block, a single block)."""
+# (queries, heads, keys) and whether the call splits the keys over a
+# workgroup's waves, on 256 CUs (test_plans.py asks the library). 260 heads of
+# 100 or more queries fill the GPU with 128-query workgroups: the step loop's
+# two-step unroll and every tail (13, 14 and 15 blocks: after the loop one or no
+# further step, then the step whose next block is the last, alternating tiles),
+# two, three and one block, whole and ragged query tiles and last blocks.
+BOTH_KERNELS = [(128, 260, 1600, False), (100, 260, 1664, False), (129, 260, 1792, False), (128, 260, 1920, False),
+                (100, 260, 130, False), (129, 260, 384, False), (200, 260, 64, False),
+                (33, 260, 1600, True), (64, 260, 1664, True), (40, 260, 1792, True), (33, 260, 1920, True),
+                (32, 260, 130, True)]
+# A few heads of enough queries for five rounds of split workgroups, many keys.
+LONG_PLAIN = (9000, 4, 16384, False)
+
+
+@pytest.mark.parametrize('nq,heads,nk,split', BOTH_KERNELS)
+def test_both_kernels_match_oracle(gpu, nq, heads, nk, split):
+    """The kernel that the whole call takes, and one head alone (always split
+    here, but for a single block), against the oracle."""
     g = torch.Generator().manual_seed(nq + nk)
-    q, k, v = _qkv(g, 1, 260, nq, nk, torch.float16)
+    q, k, v = _qkv(g, 1, heads, nq, nk, torch.float16)
     many = np_of(kernels.attention(kernels.attention_prepare(q.to(gpu), k.to(gpu), v.to(gpu)), out_dtype=torch.float32))
-    for h in (0, 259):
+    for h in (0, heads - 1):
         qh, kh, vh = (t[:, h:h + 1].contiguous() for t in (q, k, v))
         one = np_of(kernels.attention(kernels.attention_prepare(qh.to(gpu), kh.to(gpu), vh.to(gpu)),
                                       out_dtype=torch.float32))
@@ -227,3 +238,18 @@ def test_both_kernels_match_oracle(gpu, nq, nk):
         # 1e-5: the bound of test_attention_matches_oracle (hardware exp2, FP32 order)
         for out in (many[:, h:h + 1], one):
             assert np.abs(out - want).max() <= 1e-5 * np.abs(want).max()
+
+
+def test_long_rows_without_the_split(gpu):
+    """Many keys on the kernel of 128-query workgroups: the first 32 queries
+    and the ragged last ones of two heads (queries are independent, and a
+    32-row group shares its scales)."""
+    nq, heads, nk, _ = LONG_PLAIN
+    g = torch.Generator().manual_seed(nk)
+    q, k, v = _qkv(g, 1, heads, nq, nk, torch.float16)
+    out = np_of(kernels.attention(kernels.attention_prepare(q.to(gpu), k.to(gpu), v.to(gpu)), out_dtype=torch.float32))
+    for h in (0, heads - 1):
+        for a, b in ((0, 32), (nq // 32 * 32, nq)):
+            qh, kh, vh = q[:, h:h + 1, a:b].contiguous(), k[:, h:h + 1].contiguous(), v[:, h:h + 1].contiguous()
+            want = oa.kitchen_attention(oa.kitchen_prepare(_np(qh), _np(kh), _np(vh), cta_k=oa.GPU_CTA_K))
+            assert np.abs(out[:, h:h + 1, a:b] - want).max() <= 1e-5 * np.abs(want).max()

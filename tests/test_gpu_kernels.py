@@ -75,12 +75,28 @@ def test_gemm_dispatch_sweep(gpu, m, n, k):
         assert_bits_equal(np_of(got), want, f'row f16 {m}x{n}x{k} ws={workspace is None}')
 
 
-@pytest.mark.parametrize('m,n', [(4300, 4200), (6814, 5376), (353, 25000)])
-@pytest.mark.parametrize('k', [128, 256, 384, 1152, 3584])
+# More work items than CUs (on 256 of them), as (M, N, K) and the plan (tile
+# shape, K splits, items; test_plans.py asks the library for it): the operand
+# ring of each tile shape crosses tile boundaries at phases other than zero.
+# 256 x 256 (4) and 256 x 192 (3): five half-stage slots, an item of s stages
+# moves the ring by 2 s mod 5; 128 x 256 (2): three stages, s mod 3; 128 x 192
+# (1): four stages, s mod 4.
+RING_CASES = [
+    ((4300, 4200, 128), (4, 1, 289)), ((4300, 4200, 256), (4, 1, 289)), ((4300, 4200, 384), (4, 1, 289)),
+    ((4300, 4200, 1152), (4, 1, 289)), ((4300, 4200, 3584), (3, 1, 374)), ((6814, 5376, 128), (4, 1, 567)),
+    ((6814, 5376, 256), (4, 1, 567)), ((6814, 5376, 384), (4, 1, 567)), ((6814, 5376, 1152), (4, 1, 567)),
+    ((6814, 5376, 3584), (3, 1, 756)), ((6814, 5376, 3712), (3, 1, 756)),
+    ((309, 33000, 128), (2, 1, 387)), ((309, 33000, 640), (2, 1, 387)), ((309, 33000, 1280), (2, 1, 387)),
+    ((309, 33000, 1408), (2, 1, 387)), ((100, 70000, 1280), (2, 1, 274)),
+    ((100, 70000, 1408), (1, 1, 365)), ((100, 70000, 1664), (1, 1, 365)), ((100, 70000, 1792), (1, 1, 365)),
+]
+
+
+@pytest.mark.parametrize('m,n,k', [shape for shape, _ in RING_CASES] +
+                         [(353, 25000, k) for k in (128, 256, 384, 1152, 3584)])   # one round of 196 tiles
 def test_gemm_stage_ring_across_tiles(gpu, m, n, k):
-    """More output tiles of each tile shape than CUs at 1, 2, 3, 9 and 28
-    stages: the operand ring crosses tile boundaries at every phase. int32
-    sums are exact in float64 (|C| <= 3584 * 2^14 < 2^53)."""
+    """RING_CASES, int32 and fp16 epilogues. int32 sums are exact in float64
+    (|C| <= 3712 * 2^14 < 2^53)."""
     g = torch.Generator(device=gpu).manual_seed(m + n + k)
     a = torch.randint(-128, 128, (m, k), generator=g, device=gpu, dtype=torch.int8)
     b = torch.randint(-128, 128, (n, k), generator=g, device=gpu, dtype=torch.int8)
@@ -267,16 +283,29 @@ def test_gemm_stream_strided_weight_and_short_k(gpu):
         assert_bits_equal(np_of(kernels.gemm(a.to(gpu), b.to(gpu))), o.int_mm(np_of(a), np_of(b)), f'k={k}')
 
 
-@pytest.mark.parametrize('m,n,k', [(4096, 3072, 3072), (2000, 2900, 16384), (700, 3000, 1024), (353, 5120, 12800),
-                                   (353, 512, 5120)])
+# Shapes the host plans with the narrower tiles and their plans, on 256 CUs:
+# 256 x 192 tiles, 16 x 16 = 256 of them filling the GPU where 256 x 256 leaves
+# 64 CUs idle (4096 x 3072), and with K split two ways and ragged edges in M and
+# N (1500 x 2900: last tiles of 220 rows and 20 columns); 256 ragged 128 x 192
+# tiles over a long K (2000 x 2900); 128 x 256 tiles for M of a few hundred
+# rows, unsplit (700 x 3000: last tile of 60 rows), K split four (353 x 5120)
+# and eight ways (353 x 512: two tile columns, the second of 256).
+TILE_SHAPES = [((4096, 3072, 3072), (3, 1, 256)), ((1500, 2900, 16384), (3, 2, 192)),
+               ((2000, 2900, 16384), (1, 1, 256)), ((700, 3000, 1024), (2, 1, 72)),
+               ((353, 5120, 12800), (2, 4, 240)), ((353, 512, 5120), (2, 8, 48))]
+# 128 x 192 tiles: ragged in both directions (last tiles of 104 rows and 120
+# columns), K split two, four and eight ways, output rows that are not 16-byte
+# aligned, and more tiles than CUs (the four-stage ring crosses tile
+# boundaries). 200 x 1000 x 512, short enough for one launch, has 128 x 256.
+NARROW_TILE_SHAPES = [((1000, 3000, 1536), (1, 1, 128)), ((200, 1000, 512), (2, 1, 8)),
+                      ((500, 2900, 4096), (1, 2, 128)), ((200, 1000, 1024), (1, 4, 48)),
+                      ((300, 700, 16384), (1, 8, 96)), ((900, 5001, 1664), (1, 1, 216)),
+                      ((100, 70000, 1536), (1, 1, 365))]
+
+
+@pytest.mark.parametrize('m,n,k', [shape for shape, _ in TILE_SHAPES])
 def test_gemm_tile_shapes(gpu, m, n, k):
-    # Shapes the host plans with the narrower tiles, on 256 CUs: 256 x 192
-    # tiles, 16 x 16 = 256 of them filling the GPU where 256 x 256 leaves 64
-    # CUs idle (4096 x 3072), and with K split two ways and ragged edges in M
-    # and N (2000 x 2900: last tiles of 208 rows and 20 columns); 128 x 256
-    # tiles for M of a few hundred rows, unsplit (700 x 3000: last tile of 60
-    # rows), K split four (353 x 5120) and eight ways (353 x 512: two tile
-    # columns, the second of 256). Every epilogue variant.
+    # Every epilogue variant.
     print(f'tile shapes {m}x{n}x{k}', flush=True)
     g = torch.Generator().manual_seed(m + n + k)
     a = randi8(g, (m, k))
@@ -308,12 +337,8 @@ def test_gemm_tile_shapes(gpu, m, n, k):
                           f'column {out_dtype}')
 
 
-@pytest.mark.parametrize('m,n,k', [(1000, 3000, 1536), (200, 1000, 512), (900, 5001, 1664), (100, 70000, 1536)])
+@pytest.mark.parametrize('m,n,k', [shape for shape, _ in NARROW_TILE_SHAPES])
 def test_gemm_128x192_tiles(gpu, m, n, k):
-    # Shapes the host plans with 128 x 192 tiles, on 256 CUs: ragged in both
-    # directions (last tiles of 104 rows and 120 columns), K split two ways,
-    # output rows that are not 16-byte aligned, and more tiles than CUs (365:
-    # the four-stage ring crosses tile boundaries). Every epilogue variant.
     test_gemm_tile_shapes(gpu, m, n, k)
 
 

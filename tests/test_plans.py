@@ -7,6 +7,8 @@ from pathlib import Path
 import pytest
 
 import build_lib
+from test_gpu_attention import BOTH_KERNELS, LONG_PLAIN
+from test_gpu_kernels import NARROW_TILE_SHAPES, RING_CASES, TILE_SHAPES
 
 TESTS = Path(__file__).resolve().parent
 CUS = 256
@@ -37,3 +39,22 @@ def test_narrow_tiles_do_not_add_a_finishing_launch(ask, m, n, k, nb):
 @pytest.mark.parametrize('m,n,k', [(160, 512, 2304), (146, 512, 2432), (1060, 256, 3840), (126, 1280, 3584)])
 def test_narrow_tiles_split_eight_ways_only_where_that_was_the_plan(ask, m, n, k):
     assert ask('gemm', m, n, k)[:2] == (T128x256, 4)
+
+
+@pytest.mark.parametrize('shape,plan', RING_CASES + TILE_SHAPES + NARROW_TILE_SHAPES)
+def test_plans_of_the_gpu_tests(ask, shape, plan):
+    assert ask('gemm', *shape) == plan
+
+
+def test_ring_cases_cross_tile_boundaries_at_other_phases():
+    slots = {T256: (2, 5), T256x192: (2, 5), T128x256: (1, 3), T128x192: (1, 4)}
+    for nb, (units, ring) in slots.items():
+        phases = {units * (k // 128) % ring for (_, _, k), plan in RING_CASES if plan[0] == nb and plan[2] > CUS}
+        assert phases - {0}, nb
+    assert {k // 128 % 4 for (_, _, k), plan in RING_CASES if plan[0] == T128x192} == {1, 2, 3}
+
+
+@pytest.mark.parametrize('nq,heads,nk,split', BOTH_KERNELS + [LONG_PLAIN])
+def test_attention_kernels_of_the_gpu_tests(ask, nq, heads, nk, split):
+    assert ask('attention', nq, heads, nk) == (int(split),)
+    assert ask('attention', nq, 1, nk) == (int(nk > 128),) or (nq, heads, nk, split) == LONG_PLAIN
