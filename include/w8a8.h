@@ -328,6 +328,12 @@ typedef struct W8A8AttentionArgs {
   void* stream;
 } W8A8AttentionArgs;
 
+/* The kernel is chosen from nq, b * h, nk and the GPU's CU count: calls too
+ * small to fill the GPU split the keys over a workgroup's waves. The codes and
+ * probabilities are the same either way; the FP32 sums over key blocks are
+ * taken in another order, so a head computed alone and in a larger call may
+ * differ in their last bits (~1e-7 of the largest output). The same call gives
+ * the same bits every time. */
 int w8a8_attention(const W8A8AttentionArgs* args);
 
 /*

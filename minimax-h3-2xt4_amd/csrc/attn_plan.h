@@ -16,7 +16,8 @@ constexpr int kAttnWaves = 4;      // wavefronts per workgroup (one per SIMD; tw
 // x 256 15.6 / 14.0, 28 x 700 x 256 19.5 / 20.1, 20 x 1000 x 512 26.1 / 22.2,
 // 28 x 1100 x 512 28.7 / 31.0, 24 x 700 x 3000 68.7 / 65.3, 12 x 2000 x 2000
 // 52.0 / 50.4, 16 x 2000 x 2000 55.0 / 65.5. A single block has nothing to
-// split (28 x 700 x 128 9.0 / 20.2).
+// split (28 x 700 x 128 9.0 / 20.2). The FP32 sums over key blocks take another
+// order in each kernel, so a head's last bits depend on the call it is part of.
 inline bool split_wins(int64_t nq, int64_t bh, int64_t nblk, int64_t cus) {
   if (nblk < 2) return false;
   const int64_t rounds = ((nq + kAttnWaveQ - 1) / kAttnWaveQ * bh + cus - 1) / cus;

@@ -773,13 +773,16 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
 // What bounds it: at the large shapes the board's power. The products run on
 // 16x16x64 MFMAs, which sustain 4260 TOPS (2.08 GHz) from one wave per SIMD
 // on Gaussian int8 data where 32x32x32 sustains 3590 (1.73 GHz; MFMAs
-// alone), having half the accumulator traffic per product. The rest of the
-// energy feeds the operands. Against 32x32x32 with four-MFMA rows and the
-// reads and DMA bunched between them, timed in turn on one box: FC1
-// 16384x16384x3072 703 -> 644 us, FC2 16384x3072x8192 323 -> 295, QKV
-// 53504x9216x3072 1287 -> 1181, 4096x3072x3072 38.2 -> 34.1, 512x14336x4096
-// 31.8 -> 27.9 (of which the spreading of reads and DMA one to an MFMA is
-// 1..4%). MFMA pipes busy 0.65 at 1.84 GHz (0.64 at 1.74 before). Raster
+// alone; 4020 and 3410 on another box), having half the accumulator traffic
+// per product. The rest of the energy feeds the operands. Against 32x32x32
+// with four-MFMA rows and the reads and DMA bunched between them, timed in
+// turn on one box: FC1 16384x16384x3072 703 -> 644 us, FC2 16384x3072x8192 323
+// -> 295, QKV 53504x9216x3072 1287 -> 1181; 4096x3072x3072, fp16 out, 38.7 ->
+// 35.2 (with a bias 40.0 -> 36.4, bf16 45.8 -> 42.9), 512x14336x4096 32.8 ->
+// 29.8 (33.9 -> 33.6 with the weights from HBM); up to three stages of K (384)
+// within 3% either way. The spreading of reads and DMA one to an MFMA is 1..4%
+// of it. MFMA pipes busy 0.62 at 1.85 GHz in FC1 (0.61 at 1.70 before), 0.68 in
+// FC2. Raster
 // groups of 4 row tiles instead of 8 (A rows that stay in an XCD's L2) were
 // within 1% either way, and non-temporal loads of either operand 5..50%
 // slower.
@@ -792,8 +795,9 @@ __device__ __forceinline__ void load_readout_scales(const GemmParams& p, int nw,
 // its last stage issued are younger): 8 / 16 for 256 x 256 and 8 / 14 for
 // 256 x 192 tiles. The three-stage ring waits vmcnt(NA + JB) = 12 at both, the
 // four-stage ring 2 (NA + JB) = 20 and NA + JB = 10.
-// Loads return in order, so a count is exact whenever at least that many
-// younger loads exist.
+// Loads return in order, LDS DMA and loads into registers in one sequence (the
+// compiler counts them so itself), so a count is exact whenever at least that
+// many younger loads exist.
 //
 // LDS rows are 128 bytes: 16-byte chunk c of row r sits at physical chunk
 // c ^ ((r >> 1) & 7), which keeps both the DMA writes (lane i writes bytes
@@ -935,9 +939,9 @@ void gemm_i8_persistent(GemmParams p) {
   point(0);
   // The ring: unit h (the A tile of global stage h / 2 for even h, its B
   // tile for odd h) goes to slot h % kSlots. A unit is NA (A) or JB (B) DMA
-  // instructions per wave, issued in halves spread between MFMAs (a burst
+  // instructions per wave, issued one to an MFMA over a sub-step (a burst
   // of them would stall the issuing wave behind the address unit). The
-  // cursor advances after a B tile's second half; past the last stage of
+  // cursor advances after a B tile's last instruction; past the last stage of
   // the last tile it stays put and re-reads that stage into slots never
   // consumed.
   // dma_end (the cursor item's last stage + 1) is recomputed only when the
@@ -973,7 +977,7 @@ void gemm_i8_persistent(GemmParams p) {
   // v_mfma_i32_16x16x64_i8: for sub-step u (K bytes [64 u, 64 u + 64) of the
   // stage), lane (r = lane % 16, h = lane / 16) supplies row r, logical
   // chunk 4 u + h of both operands. Each wave holds an NR x 8 grid of 16x16
-  // accumulator tiles (its 128 x 32 NB quadrant).
+  // accumulator tiles (its 128 x WN quadrant).
   const int wm = BM == 128 ? 0 : wave >> 1, wn = BM == 128 ? wave : wave & 1;
   const int fr = lane & 15, fh = lane >> 4;
   const int a_row = wm * 128 * kSK + fr * kSK, b_row = wn * WN * kSK + fr * kSK;

@@ -83,11 +83,13 @@ inline int64_t plan_tiles(int64_t m, int64_t n, const GemmPlan& plan) {
 }
 
 // The plan of least modelled time for an m x n x k GEMM (k a multiple of
-// 128) on cus CUs, with at most max_split K splits. The cost is counted in
-// K = 128 stages of a 256 x 256 tile (about 1 us on the power-limited
-// clock): rounds of work items x (stages per item x the tile's relative
-// cost + the tile's epilogue and the launch's fill and drain), plus the
-// split partials' write-and-read traffic at about 6.5 TB/s. A 256 x 192
+// 128) on cus CUs, with at most max_split K splits. The cost ranks plans and
+// is no time (28 for 4096 x 3072 x 3072, which takes 36 us; 25 for 353 x 12800
+// x 5120, 35 to 41): K = 128 stages of a 256 x 256 tile, as rounds of work
+// items x (stages per item x the tile's relative cost + the tile's epilogue
+// and the launch's fill and drain), plus the split partials' write-and-read
+// traffic at about 6.5 TB/s. It knows nothing of the rate at which a CU
+// fetches lines (a 40 KB stage from HBM 0.9 us), which binds few-row shapes. A 256 x 192
 // stage costs 0.85 (0.80 of the cycles), a 128 x 256 stage 0.6 and a 128 x
 // 192 stage 0.48 with an epilogue of 6 instead of 8: fitted to the fastest
 // measured plan of shapes with M of 100..2048 rows, where 256-row tiles leave

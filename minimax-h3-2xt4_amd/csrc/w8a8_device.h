@@ -369,7 +369,25 @@ __device__ __forceinline__ void scale16(float (&v)[16]) {
 }
 
 // The 16 int8 codes of elements 16t..16t+15 (natural order), packed
-// little-endian for one 16-byte store. v_cvt_pk_u8_f32 rounds to nearest even
+// little-endian for one 16-byte store, with a tie test each (quant_round). For
+// values that were rounded to 16 bits: a ratio of two such values is a tie far
+// more often (half the row's maximum is 63.5 scales, whatever the maximum), so
+// most waves would take the second copy of quant16 below (bf16, 16384 x 3072
+// rotated, rounded and quantized: 36.2 us this way, 42.7 that way). Some
+// kernels of few waves take it too (named where they choose).
+__device__ __forceinline__ uint4 quant16_each(const float (&v)[16], float s, float rcp) {
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t b = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b = __builtin_amdgcn_cvt_pk_u8_f32(quant_round(v[4 * i + k], s, rcp) + 128.0f, k, b);
+    w[i] = b ^ 0x80808080u;
+  }
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// The same codes with one tie test for all sixteen. v_cvt_pk_u8_f32 rounds to nearest even
 // with saturation to [0, 255] and packs the byte, so the clamp to [-128, 127]
 // and the packing take one instruction per code and the XOR with 0x80 turns
 // the biased bytes into two's complement. z = x * rcp + 128 (one rounding) is
@@ -383,24 +401,6 @@ __device__ __forceinline__ void scale16(float (&v)[16]) {
 // itself (8192 x 8192 fp16 rows rotated and quantized 50.5 -> 42.9 us, a lone
 // row's workgroup 6.3 -> 5.3).
 constexpr float kNearTie = 1.25f / 65536.0f;
-
-// The codes with a test each, for values that were rounded to 16 bits: a ratio
-// of two such values is a tie far more often (half the row's maximum is 63.5
-// scales, whatever the maximum), so most waves would take the second copy
-// above (bf16, 16384 x 3072 rotated, rounded and quantized: 36.2 us this way,
-// 42.7 that way). The SwiGLU kernels of few waves to a row take it too.
-__device__ __forceinline__ uint4 quant16_each(const float (&v)[16], float s, float rcp) {
-  uint32_t w[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t b = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) b = __builtin_amdgcn_cvt_pk_u8_f32(quant_round(v[4 * i + k], s, rcp) + 128.0f, k, b);
-    w[i] = b ^ 0x80808080u;
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
-}
-
 constexpr float kWideScale = 0x1p120f;
 
 __device__ __forceinline__ uint4 quant16(const float (&v)[16], float s, float rcp) {
