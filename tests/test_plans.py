@@ -58,3 +58,9 @@ def test_ring_cases_cross_tile_boundaries_at_other_phases():
 def test_attention_kernels_of_the_gpu_tests(ask, nq, heads, nk, split):
     assert ask('attention', nq, heads, nk) == (int(split),)
     assert ask('attention', nq, 1, nk) == (int(nk > 128),) or (nq, heads, nk, split) == LONG_PLAIN
+
+
+@pytest.mark.parametrize('nq,heads,nk,split', [(2752, 6, 357, 0), (5435, 4, 364, 0), (6139, 4, 748, 0), (6139, 4, 492, 1),
+                                               (6139, 4, 1004, 1), (353, 16, 1000, 1), (700, 24, 3000, 1)])
+def test_three_rounds_split_only_full_steps(ask, nq, heads, nk, split):
+    assert ask('attention', nq, heads, nk) == (split,)
