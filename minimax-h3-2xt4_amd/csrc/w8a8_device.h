@@ -19,7 +19,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 __device__ constexpr float kR127 = 1.0f / 127.0f;
 __device__ constexpr float kScaleFloor = 1e-30f;
 __device__ constexpr float kInv16 = 1.0f / 16.0f;
-// Fast-path bound of quant1 / quant16: |y - rint(y)| below this means the
+// Fast-path bound of quant1 / quant_round: |y - rint(y)| below this means the
 // reciprocal product y = x * rcp and the IEEE quotient x / s round to the
 // same integer. rcp = 1/s is correctly rounded and the product is rounded
 // once, so |y - x/s| <= |x/s| (2^-23 + 2^-48) < 2^-16 for |x/s| < 128 (every
